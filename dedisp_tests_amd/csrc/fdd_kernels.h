@@ -130,9 +130,10 @@ hipError_t dd_fdd_contract_mfma(int prec, const float2* X, size_t Xp, const uint
                                 float xscale, float2* Y, size_t Yp, hipStream_t stream);
 
 // Phasor contraction on 16 x 16 matrix-core tiles with the real and
-// imaginary outputs of a chunk side by side along N. prec: 1 = bfloat16 with
-// hi+lo split phasors and spectra (three products), 2 = float16 (one
-// product); float32 accumulation. q: [ndm][qpitch] uint32 phase steps
+// imaginary outputs of a chunk side by side along N. prec: 0 = float32 as
+// float16 hi+lo pairs (three products), 1 = bfloat16 with hi+lo split phasors
+// and spectra (three products), 2 = float16 (one product); float32
+// accumulation; prec 0 and 2 take the xscale of dd_fdd_contract_mfma. q: [ndm][qpitch] uint32 phase steps
 // d mod nfft (qpitch a multiple of 32, >= nchan rounded up to 32, zero
 // padded); X must hold nchan rounded up to 32 channel rows, the extra rows
 // zero. mirror != 0: each workgroup takes two bins k, k+1 <= nfft/4 and their
@@ -141,15 +142,14 @@ hipError_t dd_fdd_contract_mfma(int prec, const float2* X, size_t Xp, const uint
 // (e^{+2 pi i m/nfft}, mirror only) each row instead holds the packed
 // half-length spectrum the inverse transform starts from,
 // Zu[k] = (Y[k] + conj Y[M-k]) + i e^{2 pi i k/nfft} (Y[k] - conj Y[M-k]), k < M.
-// prec 0 = float32 (v_mfma_f32_16x16x4_f32). With dmlist (ndm floats) and
+// With dmlist (ndm floats) and
 // delay32 (the delay table, nchan rounded up to 32 entries, zero padded) the
 // integer delays are computed in the kernel as (int)(dm * delay[c]) and q is
 // not read.
 // cfg selects the workgroup shape: 0 = 8 waves of 2 16-row DM tiles and 4
 // bin slots; 1 = 4 waves of 4 DM tiles and 2 bin slots (half the B-operand
 // LDS reads per product, two workgroups per CU); 2 = the software-pipelined
-// form of 0 (bfloat16 / float16 with dmlist; a K-step's spectra within 32-bit
-// element offsets). blocked != 0 (cfg 2 with mirror and ph_packed, nfft <=
+// form of 0 (with dmlist; a K-step's spectra within 32-bit element offsets). blocked != 0 (cfg 2 with mirror and ph_packed, nfft <=
 // 65536): X and the packed output in the bin-block layout of
 // dd_fdd_forward_split (Xp and Yp unused).
 hipError_t dd_fdd_contract_mfma16(int prec, int mirror, const float2* X, size_t Xp, const uint32_t* q,

@@ -1,6 +1,6 @@
 // gfx950 phasor contraction of the FDD path on 16 x 16 matrix-core tiles, re
-// and im side by side along N (float32, bfloat16 three-product and float16
-// single-product forms).
+// and im side by side along N (float32 and bfloat16 as hi + lo pairs with
+// three products, float16 with a single product).
 //
 // For every Fourier bin k the dedispersed spectra are a complex GEMM
 //   Y_k[dm][chunk] = sum_c P_k[dm][c] X_k[c][chunk],  P_k[dm][c] = e^{+2 pi i k d(dm,c)/nfft}
@@ -24,12 +24,21 @@
 // exact integer (k*q) mod nfft with q = d mod nfft (q[dm][c], uint32), and
 // v_cos_f32 / v_sin_f32 take it in revolutions, (k*q mod nfft)/nfft, exact in
 // float for nfft <= 2^24.
-// float32: v_mfma_f32_16x16x4_f32, one phasor component per lane;
-// bfloat16 (v_mfma_f32_16x16x32_bf16): phasors and spectra split into
-// truncated hi + rounded lo, products Ph Xh + Ph Xl + Pl Xh (the remainder
-// x - hi is exact in float32); float16 (v_mfma_f32_16x16x32_f16):
-// round-to-nearest, spectra scaled by a power of two into the float16 range.
-// Float32 accumulation.
+// bfloat16 (v_mfma_f32_16x16x32_bf16): phasors and spectra split into hi +
+// rounded lo, products Ph Xh + Ph Xl + Pl Xh (the remainder x - hi is exact in
+// float32); float16 (v_mfma_f32_16x16x32_f16): round-to-nearest, spectra
+// scaled by a power of two into the float16 range. Float32 accumulation.
+// float32: the bfloat16 form's three products on float16 hi + lo pairs, which
+// carry 22 of the 24 significand bits: the rounding of lo and the dropped lo lo
+// product are each about 2^-24 of a term (rms), below the float32 rounding of
+// the sums. The scale keeps |X| <= 2^15; float16 subnormals then resolve
+// 2^-39 of the largest possible spectrum value, under the transforms' own
+// rounding (2^-24 of rms(x) sqrt(nfft), against the bound max(x) nfft) for every
+// segment length. Against float64 the output is off by 4.9e-7 (1024 ch x
+// 2^19 samples x 1000 DMs) where float32 matrix products with the
+// three-product complex multiply are off by 7.5e-7; at 1024 ch x 2048 DMs x 23
+// chunks of 65536 it takes 39.7 ms instead of 120 (float16 products run at 16
+// times the float32 rate, and three of them stand for one).
 //
 // Operand layout: lane l of A holds DM row l%16 and channels 8*(l/16) .. +7 of
 // the K-step; lane l of B holds column l%16 and the same channels, so the sum
@@ -99,6 +108,30 @@ __device__ __forceinline__ uint32_t pack_f16x2(float a, float b)
     return __builtin_bit_cast(uint32_t, v);
 }
 
+// hi: the round-to-nearest float16 of a (low half) and b (high half); lo: the
+// rounded float16 of the exact remainders a - hi(a), b - hi(b) (one mixed
+// fused multiply-add each). hi + lo carries 22 significand bits.
+__device__ __forceinline__ void split_f16x2(float a, float b, uint32_t& hi, uint32_t& lo)
+{
+    asm volatile("" : "+v"(a), "+v"(b));
+    const f16x2 h = {(_Float16)a, (_Float16)b};
+    const float ra = __builtin_fmaf((float)h[0], -1.0f, a);
+    const float rb = __builtin_fmaf((float)h[1], -1.0f, b);
+    hi = __builtin_bit_cast(uint32_t, h);
+    lo = pack_f16x2(ra, rb);
+}
+
+// The matrix product of a form: float16 operands (float32's split form and
+// float16) or bfloat16.
+__device__ __forceinline__ f32x4 mfma(f16x8 a, f16x8 b, f32x4 c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
 // Staged spectra planes per form and bytes per element; a staged column
 // holds the 32 channels of a K-step plus 16 bytes, so that the 16-byte reads
 // of 8 consecutive columns cover all banks (column strides 80 and 144 bytes
@@ -106,9 +139,9 @@ __device__ __forceinline__ uint32_t pack_f16x2(float a, float b)
 template <int PREC>
 struct Planes;
 template <>
-struct Planes<0> {  // float32: [Xr|Xi], [-Xi|Xr]
-    static constexpr int N = 2, ELEM = 4;
-    using V = float;
+struct Planes<0> {  // float32 as float16 hi + lo: the planes of the bfloat16 form
+    static constexpr int N = 4, ELEM = 2;
+    using V = f16x8;
 };
 template <>
 struct Planes<1> {  // bfloat16: [Xr|Xi] hi, [Xr|Xi] lo, [-Xi|Xr] hi, [-Xi|Xr] lo
@@ -164,7 +197,7 @@ __global__ __launch_bounds__(WAVES * 64, 512 / (WAVES * 64)) void fdd_mfma16_k(
     float2* __restrict__ Y, size_t Yp, uint32_t nbb, uint32_t ndb, const float2* __restrict__ zph,
     const float* __restrict__ dmlist, const float* __restrict__ dtab)
 {
-    static_assert(!PIPE || (PREC != 0 && NS == 4 && WAVES == 8), "pipelined form: bfloat16 / float16");
+    static_assert(!PIPE || (NS == 4 && WAVES == 8), "pipelined form: 8 waves, 4 slots");
     static_assert(!BLK || (PIPE && MIRROR), "bin-block layout: pipelined form with mirror bins");
     constexpr int NT = WAVES * 64;        // threads
     constexpr int DPB = WAVES * MT * 16;  // DMs per workgroup
@@ -237,14 +270,12 @@ __global__ __launch_bounds__(WAVES * 64, 512 / (WAVES * 64)) void fdd_mfma16_k(
         const float xr0 = x0.x * sscale[u], xi0 = x0.y * sscale[u];
         const float xr1 = x1.x * sscale[u], xi1 = x1.y * sscale[u];
         char* b = buf + soff[u];
-        if constexpr (PREC == 0) {
-            *reinterpret_cast<float2*>(b) = make_float2(xr0, xr1);
-            *reinterpret_cast<float2*>(b + 8 * COLB) = make_float2(xi0, xi1);
-            *reinterpret_cast<float2*>(b + G::PSTR) = make_float2(-xi0, -xi1);
-            *reinterpret_cast<float2*>(b + G::PSTR + 8 * COLB) = make_float2(xr0, xr1);
-        } else if constexpr (PREC == 1) {
+        if constexpr (PREC != 2) {
             uint32_t rh, rl, ih, il;
-            if constexpr (PIPE) {
+            if constexpr (PREC == 0) {
+                split_f16x2(xr0, xr1, rh, rl);
+                split_f16x2(xi0, xi1, ih, il);
+            } else if constexpr (PIPE) {
                 split_bf16x2_rn(xr0, xr1, rh, rl, dsel);
                 split_bf16x2_rn(xi0, xi1, ih, il, dsel);
             } else {
@@ -360,78 +391,27 @@ __global__ __launch_bounds__(WAVES * 64, 512 / (WAVES * 64)) void fdd_mfma16_k(
                     }
             }
 
-            if constexpr (PREC == 0) {
-                // float32: A is one phasor component per lane and 16 x 16 x 4
-                // MFMA; MFMA e of a K-step sums channels 8g + e of the lane groups
-    #pragma unroll
-                for (int b = 0; b < NDIR; ++b) {
-                    const uint32_t kb = k0 + b;
-                    float pr[MT][8], pim[MT][8];
-    #pragma unroll
-                    for (int mt = 0; mt < MT; ++mt)
-    #pragma unroll
-                        for (int e = 0; e < 8; ++e) {
-                            const uint32_t qq = qc[mt][e >> 2][e & 3];
-                            const float a = (float)(__umul24(kb, qq) & mask) * inv;
-                            pr[mt][e] = __builtin_amdgcn_cosf(a);
-                            pim[mt][e] = __builtin_amdgcn_sinf(a);
-                        }
-    #pragma unroll
-                    for (int pass = 0; pass < (MIRROR ? 2 : 1); ++pass) {
-                        const int s = pass ? NDIR + b : b;
-                        if (pass) {
-                            // re' = (-1)^d re, im' = -(-1)^d im
-    #pragma unroll
-                            for (int mt = 0; mt < MT; ++mt)
-    #pragma unroll
-                                for (int e = 0; e < 8; ++e) {
-                                    const uint32_t sg = (qc[mt][e >> 2][e & 3] & 1u) << 31;
-                                    pr[mt][e] = __builtin_bit_cast(float, fbits(pr[mt][e]) ^ sg);
-                                    pim[mt][e] = __builtin_bit_cast(float, fbits(pim[mt][e]) ^ sg ^ 0x80000000u);
-                                }
-                        }
-                        const char* sb = cur + s * G::SSTR + b_off;
-    #pragma unroll
-                        for (int t = 0; t < NTL; ++t) {
-                            float xr[8], xi[8];
-                            *reinterpret_cast<float4*>(xr) = *reinterpret_cast<const float4*>(sb + t * 16 * COLB);
-                            *reinterpret_cast<float4*>(xr + 4) =
-                                *reinterpret_cast<const float4*>(sb + t * 16 * COLB + 16);
-                            *reinterpret_cast<float4*>(xi) =
-                                *reinterpret_cast<const float4*>(sb + G::PSTR + t * 16 * COLB);
-                            *reinterpret_cast<float4*>(xi + 4) =
-                                *reinterpret_cast<const float4*>(sb + G::PSTR + t * 16 * COLB + 16);
-    #pragma unroll
-                            for (int e = 0; e < 8; ++e)
-    #pragma unroll
-                                for (int mt = 0; mt < MT; ++mt) {
-                                    acc[s][mt][t] =
-                                        __builtin_amdgcn_mfma_f32_16x16x4f32(pr[mt][e], xr[e], acc[s][mt][t], 0, 0, 0);
-                                    acc[s][mt][t] =
-                                        __builtin_amdgcn_mfma_f32_16x16x4f32(pim[mt][e], xi[e], acc[s][mt][t], 0, 0, 0);
-                                }
-                        }
-                    }
-                }
-            } else {
-        #pragma unroll
+#pragma unroll
                 for (int b = 0; b < NDIR; ++b) {
                     const uint32_t kb = k0 + b;
                     // phasor planes of bin kb for the two DM tiles
                     uint32_t A[MT][PL::N][4];
-        #pragma unroll
+#pragma unroll
                     for (int mt = 0; mt < MT; ++mt)
-        #pragma unroll
+#pragma unroll
                         for (int j = 0; j < 4; ++j) {
                             float cr[2], ci[2];
-        #pragma unroll
+#pragma unroll
                             for (int h = 0; h < 2; ++h) {
                                 const uint32_t qq = qc[mt][j >> 1][2 * (j & 1) + h];
                                 const float a = (float)(__umul24(kb, qq) & mask) * inv;
                                 cr[h] = __builtin_amdgcn_cosf(a);
                                 ci[h] = __builtin_amdgcn_sinf(a);
                             }
-                            if constexpr (PREC == 1) {
+                            if constexpr (PREC == 0) {
+                                split_f16x2(cr[0], cr[1], A[mt][0][j], A[mt][1][j]);
+                                split_f16x2(ci[0], ci[1], A[mt][2][j], A[mt][3][j]);
+                            } else if constexpr (PREC == 1) {
                                 split_bf16x2(cr[0], cr[1], A[mt][0][j], A[mt][1][j]);
                                 split_bf16x2(ci[0], ci[1], A[mt][2][j], A[mt][3][j]);
                             } else {
@@ -440,64 +420,63 @@ __global__ __launch_bounds__(WAVES * 64, 512 / (WAVES * 64)) void fdd_mfma16_k(
                             }
                         }
                     // the direct slot, then (MIRROR) its mirror with the signs flipped
-        #pragma unroll
+#pragma unroll
                     for (int pass = 0; pass < (MIRROR ? 2 : 1); ++pass) {
                         const int s = pass ? NDIR + b : b;
                         if (pass) {
-        #pragma unroll
+#pragma unroll
                             for (int mt = 0; mt < MT; ++mt)
-        #pragma unroll
+#pragma unroll
                                 for (int j = 0; j < 4; ++j) {
                                     // re' = (-1)^d re, im' = -(-1)^d im
-        #pragma unroll
+#pragma unroll
                                     for (int pl = 0; pl < PL::N; ++pl)
                                         A[mt][pl][j] ^= smask[mt][j] ^ ((pl >= PL::N / 2) ? 0x80008000u : 0u);
                                 }
                         }
                         V a[MT][PL::N];
-        #pragma unroll
+#pragma unroll
                         for (int mt = 0; mt < MT; ++mt)
-        #pragma unroll
+#pragma unroll
                             for (int pl = 0; pl < PL::N; ++pl) a[mt][pl] = __builtin_bit_cast(V, A[mt][pl]);
                         const char* sb = cur + s * G::SSTR + b_off;
-        #pragma unroll
+#pragma unroll
                         for (int t = 0; t < NTL; ++t) {
                             V x[PL::N];
-        #pragma unroll
+#pragma unroll
                             for (int pl = 0; pl < PL::N; ++pl)
                                 x[pl] = *reinterpret_cast<const V*>(sb + pl * G::PSTR + t * 16 * COLB);
-                            if constexpr (PREC == 1) {
+                            if constexpr (PREC != 2) {
                                 // planes: 0 Ar hi, 1 Ar lo, 2 Ai hi, 3 Ai lo; x: 0 BR hi, 1 BR lo, 2 BI hi, 3 BI lo
-        #pragma unroll
+#pragma unroll
                                 for (int mt = 0; mt < MT; ++mt)
-                                    acc[s][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt][0], x[0], acc[s][mt][t], 0, 0, 0);
-        #pragma unroll
+                                    acc[s][mt][t] = mfma(a[mt][0], x[0], acc[s][mt][t]);
+#pragma unroll
                                 for (int mt = 0; mt < MT; ++mt)
-                                    acc[s][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt][2], x[2], acc[s][mt][t], 0, 0, 0);
-        #pragma unroll
+                                    acc[s][mt][t] = mfma(a[mt][2], x[2], acc[s][mt][t]);
+#pragma unroll
                                 for (int mt = 0; mt < MT; ++mt)
-                                    acc[s][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt][0], x[1], acc[s][mt][t], 0, 0, 0);
-        #pragma unroll
+                                    acc[s][mt][t] = mfma(a[mt][0], x[1], acc[s][mt][t]);
+#pragma unroll
                                 for (int mt = 0; mt < MT; ++mt)
-                                    acc[s][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt][2], x[3], acc[s][mt][t], 0, 0, 0);
-        #pragma unroll
+                                    acc[s][mt][t] = mfma(a[mt][2], x[3], acc[s][mt][t]);
+#pragma unroll
                                 for (int mt = 0; mt < MT; ++mt)
-                                    acc[s][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt][1], x[0], acc[s][mt][t], 0, 0, 0);
-        #pragma unroll
+                                    acc[s][mt][t] = mfma(a[mt][1], x[0], acc[s][mt][t]);
+#pragma unroll
                                 for (int mt = 0; mt < MT; ++mt)
-                                    acc[s][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt][3], x[2], acc[s][mt][t], 0, 0, 0);
+                                    acc[s][mt][t] = mfma(a[mt][3], x[2], acc[s][mt][t]);
                             } else {
-        #pragma unroll
+#pragma unroll
                                 for (int mt = 0; mt < MT; ++mt)
-                                    acc[s][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[mt][0], x[0], acc[s][mt][t], 0, 0, 0);
-        #pragma unroll
+                                    acc[s][mt][t] = mfma(a[mt][0], x[0], acc[s][mt][t]);
+#pragma unroll
                                 for (int mt = 0; mt < MT; ++mt)
-                                    acc[s][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[mt][1], x[1], acc[s][mt][t], 0, 0, 0);
+                                    acc[s][mt][t] = mfma(a[mt][1], x[1], acc[s][mt][t]);
                             }
                         }
                     }
                 }
-            }
 
             if (more) store_x(xs + ((ks + 1) & 1) * BUF);
             __syncthreads();
@@ -539,7 +518,10 @@ __global__ __launch_bounds__(WAVES * 64, 512 / (WAVES * 64)) void fdd_mfma16_k(
                 cr[h] = __builtin_amdgcn_cosf(x);
                 ci[h] = __builtin_amdgcn_sinf(x);
             }
-            if constexpr (PREC == 1) {
+            if constexpr (PREC == 0) {
+                split_f16x2(cr[0], cr[1], A[mt][0][j], A[mt][1][j]);
+                split_f16x2(ci[0], ci[1], A[mt][2][j], A[mt][3][j]);
+            } else if constexpr (PREC == 1) {
                 split_bf16x2_rn(cr[0], cr[1], A[mt][0][j], A[mt][1][j], dsel);
                 split_bf16x2_rn(ci[0], ci[1], A[mt][2][j], A[mt][3][j], dsel);
             } else {
@@ -561,33 +543,33 @@ __global__ __launch_bounds__(WAVES * 64, 512 / (WAVES * 64)) void fdd_mfma16_k(
             for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
                 for (int pl = 0; pl < PL::N; ++pl) a[mt][pl] = __builtin_bit_cast(V, A[mt][pl]);
-            if constexpr (PREC == 1) {
+            if constexpr (PREC != 2) {
                 // planes: 0 Ar hi, 1 Ar lo, 2 Ai hi, 3 Ai lo; x: 0 BR hi, 1 BR lo, 2 BI hi, 3 BI lo
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    acc[s][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt][0], x[0], acc[s][mt][t], 0, 0, 0);
+                    acc[s][mt][t] = mfma(a[mt][0], x[0], acc[s][mt][t]);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    acc[s][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt][2], x[2], acc[s][mt][t], 0, 0, 0);
+                    acc[s][mt][t] = mfma(a[mt][2], x[2], acc[s][mt][t]);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    acc[s][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt][0], x[1], acc[s][mt][t], 0, 0, 0);
+                    acc[s][mt][t] = mfma(a[mt][0], x[1], acc[s][mt][t]);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    acc[s][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt][2], x[3], acc[s][mt][t], 0, 0, 0);
+                    acc[s][mt][t] = mfma(a[mt][2], x[3], acc[s][mt][t]);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    acc[s][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt][1], x[0], acc[s][mt][t], 0, 0, 0);
+                    acc[s][mt][t] = mfma(a[mt][1], x[0], acc[s][mt][t]);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    acc[s][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt][3], x[2], acc[s][mt][t], 0, 0, 0);
+                    acc[s][mt][t] = mfma(a[mt][3], x[2], acc[s][mt][t]);
             } else {
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    acc[s][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[mt][0], x[0], acc[s][mt][t], 0, 0, 0);
+                    acc[s][mt][t] = mfma(a[mt][0], x[0], acc[s][mt][t]);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    acc[s][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[mt][1], x[1], acc[s][mt][t], 0, 0, 0);
+                    acc[s][mt][t] = mfma(a[mt][1], x[1], acc[s][mt][t]);
             }
         };
         // The spectra are staged in two halves: items [0, IPT/2) loaded at the
@@ -861,7 +843,7 @@ extern "C" hipError_t dd_fdd_contract_mfma16(int prec, int mirror, const float2*
         nfft > (size_t(1) << 18) || (nfft & (nfft - 1)) || (!blocked && Xp < nfft / 2 + 1))
         return hipErrorInvalidValue;
     if (prec != 0 && prec != 1 && prec != 2) return hipErrorInvalidValue;
-    if (cfg < 0 || cfg > 2 || (cfg == 2 && (prec == 0 || !dmlist))) return hipErrorInvalidValue;
+    if (cfg < 0 || cfg > 2 || (cfg == 2 && !dmlist)) return hipErrorInvalidValue;
     if (blocked && (cfg != 2 || !mirror || !ph_packed || nfft > 65536)) return hipErrorInvalidValue;
     // the pipelined form addresses the spectra of a K-step by 32-bit element offsets
     const size_t rowp = blocked ? nfft / 2 + 4 : Xp;
@@ -886,8 +868,8 @@ extern "C" hipError_t dd_fdd_contract_mfma16(int prec, int mirror, const float2*
                        xscale, yscale, Y, Yp, nbb, ndb, ph_packed, dmlist, delay32)
 #define DD_M16_C(P, T, MI)                                                               \
     if (cfg == 1) DD_M16(P, T, MI, 4, 4, 2, false, false);                               \
-    else if (cfg == 2 && blocked) DD_M16(P, T, MI, 8, 2, 4, P != 0, P != 0 && MI);       \
-    else if (cfg == 2) DD_M16(P, T, MI, 8, 2, 4, P != 0, false);                         \
+    else if (cfg == 2 && blocked) DD_M16(P, T, MI, 8, 2, 4, true, MI);       \
+    else if (cfg == 2) DD_M16(P, T, MI, 8, 2, 4, true, false);                         \
     else DD_M16(P, T, MI, 8, 2, 4, false, false);
 #define DD_M16_T(P, MI)                    \
     switch (ntl) {                         \

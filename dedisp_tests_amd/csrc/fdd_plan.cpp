@@ -112,11 +112,12 @@ bool env_flag(const char* name)
     return s && std::atoi(s) != 0;
 }
 
-// The contraction kernel of a precision: the bfloat16 and float16 forms run
-// on 16 x 16 x 32 tiles with re/im along N (DEDISP_FDD_MFMA32=1 selects the
-// 32 x 32 tile kernel instead), float32 on 32 x 32 x 2 tiles
-// (DEDISP_FDD_FP32_TILE16=1: 16 x 16 x 4 tiles with re/im along N), and
-// DEDISP_FDD_VALU=1 the float32 vector-ALU form.
+// The contraction kernel of a precision: every form runs on 16 x 16 x 32 tiles
+// with re/im along N, float32 as float16 hi + lo pairs (1024 ch x 2048 DMs x
+// 23 chunks of 65536: 39.7 ms against 120 ms on float32 matrix products, and
+// nearer the float64 result). DEDISP_FDD_MFMA32=1 selects the 32 x 32 tile
+// kernel instead (DEDISP_FDD_FP32_TILE16=1 keeps float32 on 16 x 16 tiles),
+// and DEDISP_FDD_VALU=1 the float32 vector-ALU form.
 // The autotuner's choices (FDDGPUPlan::autotune) replace these defaults for
 // the precision they were timed with; the environment variables override both.
 enum class Contraction { VALU, MFMA32, MFMA16 };
@@ -130,7 +131,6 @@ Contraction contraction_kind(const FDDState& st)
     if (st.precision == DEDISP_AMD_FDD_FP32) {
         if (env_flag("DEDISP_FDD_VALU")) return Contraction::VALU;
         if (env_flag("DEDISP_FDD_FP32_TILE16")) return Contraction::MFMA16;
-        return (t && st.tuned_form != 3) ? Contraction::MFMA16 : Contraction::MFMA32;
     }
     if (env_flag("DEDISP_FDD_MFMA32")) return Contraction::MFMA32;
     return (t && st.tuned_form == 3) ? Contraction::MFMA32 : Contraction::MFMA16;
@@ -403,9 +403,9 @@ size_t FDDGPUPlan::segment_length(const size_t* nsc, size_t n) const
 
 // Phase tables of segment length nfft: e^{2 pi i m/nfft} for the transforms
 // (and the 65536-entry table of the on-chip engine when segments are split)
-// and, for the matrix-core contraction (valu false), the phase steps
-// d mod nfft. Returns the float16 spectrum scale.
-float FDDGPUPlan::prepare_phasors(size_t nfft, bool valu)
+// and, for the contraction forms that read them, the phase steps d mod nfft.
+// Returns the spectrum scale of the forms on float16 products.
+float FDDGPUPlan::prepare_phasors(size_t nfft, unsigned in_nbits)
 {
     FDDState& st = *m_state;
     hipStream_t stream = m_ctx->exec;
@@ -437,7 +437,9 @@ float FDDGPUPlan::prepare_phasors(size_t nfft, bool valu)
     }
     // phase steps of the matrix-core contraction: q = d mod nfft (phases in
     // units of 1/nfft)
-    if (!valu && (st.q32_version != m_tables_version || st.q32_nfft != nfft)) {
+    const Contraction kind = contraction_kind(st);
+    const bool qtable = kind == Contraction::MFMA32 || (kind == Contraction::MFMA16 && env_flag("DEDISP_FDD_QTABLE"));
+    if (qtable && (st.q32_version != m_tables_version || st.q32_nfft != nfft)) {
         const size_t qpitch = round_up(nchan, 32);
         std::vector<uint32_t> q(ndm * qpitch, 0);
         for (size_t i = 0; i < ndm; ++i)
@@ -450,11 +452,12 @@ float FDDGPUPlan::prepare_phasors(size_t nfft, bool valu)
         st.q32_nfft = nfft;
         st.q32_version = m_tables_version;
     }
-    // float16 spectra: |X| <= nfft * 127.5 * max scale; a power of two brings
-    // that bound to at most 2^15 (float16 max 65504)
+    // float16 products (the float16 form and float32's hi + lo form): |X| <=
+    // nfft * (2^nbits - 1)/2 * max scale; a power of two brings that bound to
+    // at most 2^15 (float16 max 65504)
     float xscale = 1.f;
-    if (st.precision == DEDISP_AMD_FDD_FP16 && st.max_scale > 0.f) {
-        const double bound = (double)nfft * 127.5 * (double)st.max_scale;
+    if (st.precision != DEDISP_AMD_FDD_BF16 && kind != Contraction::VALU && st.max_scale > 0.f) {
+        const double bound = (double)nfft * 0.5 * (double)((1u << in_nbits) - 1u) * (double)st.max_scale;
         xscale = (float)std::ldexp(1.0, (int)std::floor(std::log2(32768.0 / bound)));
     }
     return xscale;
@@ -480,33 +483,32 @@ int m16cfg_env()
 }
 
 // Workgroup shape of the 16 x 16 tile kernel: 2, the software-pipelined form
-// (8 waves of 2 DM tiles, 4 bin slots), for bfloat16 and float16 with the
-// delays computed in the kernel while a K-step's spectra stay within 32-bit
-// element offsets; else 0 (8 waves of 2 DM tiles, 4 slots). DEDISP_FDD_M16CFG
-// forces 0, 1 (4 waves of 4 DM tiles, 2 slots) or 2 where it applies.
+// (8 waves of 2 DM tiles, 4 bin slots), with the delays computed in the kernel
+// while a K-step's spectra stay within 32-bit element offsets; else 0 (8 waves
+// of 2 DM tiles, 4 slots). DEDISP_FDD_M16CFG forces 0, 1 (4 waves of 4 DM
+// tiles, 2 slots) or 2 where it applies.
 int mfma16_cfg(const FDDState& st, size_t nchunk, size_t Xp)
 {
-    const bool pipe = st.precision != DEDISP_AMD_FDD_FP32 && !env_flag("DEDISP_FDD_QTABLE") &&
-                      32 * nchunk * Xp + Xp < (size_t(1) << 32);
+    const bool pipe = !env_flag("DEDISP_FDD_QTABLE") && 32 * nchunk * Xp + Xp < (size_t(1) << 32);
     const int e = m16cfg_env();
     if (e == 0 || e == 1 || (e == 2 && pipe)) return e;
+    if (st.precision == DEDISP_AMD_FDD_FP32) return pipe ? 2 : 0;
     if (tuned(st) && (st.tuned_form == 0 || st.tuned_form == 1 || (st.tuned_form == 2 && pipe)))
         return st.tuned_form;
     return pipe ? 2 : 0;
 }
 
 // Whether the 16 x 16 tile kernel pairs each bin with its mirror
-// (DEDISP_FDD_MIRROR=0/1 forces it): by default for bfloat16 and float16,
-// whose mirror phasors save a cosine, a sine (and the hi/lo split) for half
-// the bins and which then run in the bin-block layout (1024 ch x 2048 DMs x
-// 23 chunks of 65536: float16 21.2 ms against 28.7 ms on four consecutive
-// bins); not for float32 (117.1 ms on consecutive bins against 119.5 ms).
+// (DEDISP_FDD_MIRROR=0/1 forces it): by default, since mirror phasors save a
+// cosine, a sine (and the hi/lo split) for half the bins and the kernel then
+// runs in the bin-block layout (1024 ch x 2048 DMs x 23 chunks of 65536:
+// float16 21.2 ms against 28.7 ms on four consecutive bins).
 bool mfma16_mirror(const FDDState& st)
 {
     const char* s = std::getenv("DEDISP_FDD_MIRROR");
     if (s) return std::atoi(s) != 0;
     if (tuned(st) && st.tuned_mirror >= 0) return st.tuned_mirror != 0;
-    return st.precision != DEDISP_AMD_FDD_FP32;
+    return true;
 }
 
 bool contraction_packs(const FDDState& st)
@@ -556,8 +558,9 @@ void contract(FDDState& st, size_t nchan, size_t b0, size_t nb, size_t nchunk, s
         // delays from the DM list and delay table in the kernel
         // (DEDISP_FDD_QTABLE=1: read from the phase-step table instead)
         DD_HIP(dd_fdd_contract_mfma16((int)st.precision, mfma16_mirror(st), st.d_Z.as<float2>(), Xp,
-                                      st.d_q32.as<uint32_t>() + b0 * st.qpitch32, st.qpitch32, nb, nchan, nchunk,
-                                      nfft, xscale, st.d_Y.as<float2>(), Yp,
+                                      env_flag("DEDISP_FDD_QTABLE") ? st.d_q32.as<uint32_t>() + b0 * st.qpitch32
+                                                                    : nullptr,
+                                      st.qpitch32, nb, nchan, nchunk, nfft, xscale, st.d_Y.as<float2>(), Yp,
                                       contraction_packs(st) ? st.d_ph.as<float2>() : nullptr,
                                       env_flag("DEDISP_FDD_QTABLE") ? nullptr : st.d_dm32.as<float>() + b0,
                                       env_flag("DEDISP_FDD_QTABLE") ? nullptr : st.d_delay32.as<float>(),
@@ -622,8 +625,7 @@ void FDDGPUPlan::execute_fdd(size_type nsamps, const byte_type* in, size_type in
     const size_t M = nfft / 2;
     const size_t Xp = M + 64, Yp = M + 64;  // bins 0..M, rows 512-byte aligned
 
-    const bool valu = env_flag("DEDISP_FDD_VALU") && st.precision == DEDISP_AMD_FDD_FP32;
-    const float xscale = prepare_phasors(nfft, valu);
+    const float xscale = prepare_phasors(nfft, (unsigned)in_nbits);
     const float2* ph = st.d_ph.as<float2>();
 
     // ---- input ----
@@ -810,8 +812,7 @@ void FDDGPUPlan::execute_batch(size_type nbeams, const size_type* nsamps, const 
     const size_t good = (nfft - dmax) & ~size_t(1);
     const size_t M = nfft / 2;
     const size_t Xp = M + 64, Yp = M + 64;
-    const bool valu = env_flag("DEDISP_FDD_VALU") && st.precision == DEDISP_AMD_FDD_FP32;
-    const float xscale = prepare_phasors(nfft, valu);
+    const float xscale = prepare_phasors(nfft, (unsigned)in_nbits);
     const float2* ph = st.d_ph.as<float2>();
     const size_t nchan_pad = padded_channels(nchan);
 
@@ -874,7 +875,7 @@ void FDDGPUPlan::execute_batch(size_type nbeams, const size_type* nsamps, const 
 
     // device pointers: a captured graph per batch (lengths, pointers, segment
     // length, precision, tables and buffers), replayed while they stay the same
-    std::vector<uint64_t> key = {nbeams, in_nbits, nfft, (uint64_t)st.precision, valu ? 1u : 0u,
+    std::vector<uint64_t> key = {nbeams, in_nbits, nfft, (uint64_t)st.precision,
                                  m_tables_version, max_chunks, dm_batch, __builtin_bit_cast(uint32_t, xscale),
                                  (uint64_t)st.d_rows.ptr, (uint64_t)st.d_Z.ptr, (uint64_t)st.d_Y.ptr,
                                  (uint64_t)st.d_q32.ptr, (uint64_t)st.d_ph.ptr, (uint64_t)st.d_ph64k.ptr,

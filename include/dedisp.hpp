@@ -255,7 +255,7 @@ private:
                      unsigned flags, bool fourier);
     void prepare_tables();
     size_t segment_length(const size_t* nsc, size_t n) const;
-    float prepare_phasors(size_t nfft, bool valu);
+    float prepare_phasors(size_t nfft, unsigned in_nbits);
 
     std::unique_ptr<FDDState> m_state;
 };

@@ -29,7 +29,9 @@ typedef enum {
 } dedisp_amd_fdd_output;
 
 /* Arithmetic of the FDD phasor contraction.
- *  FP32: plain float32 complex multiply-accumulate (the drop-in form);
+ *  FP32: complex multiply-accumulate to float32 accuracy (the drop-in form):
+ *        float16 MFMA with float32 accumulation on hi+lo split phasors and
+ *        spectra (22 significand bits, three-product compensation);
  *  BF16: bfloat16 MFMA with float32 accumulation, split hi+lo phasors and
  *        spectra (three-product compensation);
  *  FP16: float16 MFMA with float32 accumulation, per-channel spectrum
@@ -215,9 +217,11 @@ typedef struct {
     unsigned    candidates;   /* configurations timed */
     /* FDD contraction at that segment length: fdd_form 0, 1, 2 = the 16 x 16
      * tile kernel with 8 waves, 4 waves, software-pipelined 8 waves; 3 = the
-     * 32 x 32 tile kernel. fdd_mirror: bins paired with their mirrors (1) or
-     * consecutive (0); fdd_layout: spectra in bin blocks (1) or rows (0);
-     * -1 where the form has no such choice. 0 for TDD plans. */
+     * 32 x 32 tile kernel (float32 plans: 0 stands for the 16 x 16 tile kernel
+     * in its best shape, 3 for float32 products on 32 x 32 tiles). fdd_mirror:
+     * bins paired with their mirrors (1) or consecutive (0); fdd_layout:
+     * spectra in bin blocks (1) or rows (0); -1 where the form has no such
+     * choice. 0 for TDD plans. */
     int         fdd_form, fdd_mirror, fdd_layout;
 } dedisp_amd_tuning;
 

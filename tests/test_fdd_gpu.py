@@ -214,6 +214,41 @@ def test_fdd_forms_ragged_channels_many_chunks(dd, orc, prec):
     assert rel_l2(out, ref) < PREC_TOL[prec]
 
 
+@pytest.mark.parametrize("nbits,kind", [(8, "noise"), (8, "saturated"), (8, "faint"), (8, "tone"), (8, "impulse"),
+                                        (4, "noise"), (2, "noise"), (1, "noise")])
+@pytest.mark.parametrize("nfft", [8192, 65536, 262144])
+def test_fdd_fp32_rounds_as_float32(dd, orc, nfft, nbits, kind):
+    """The float32 form multiplies float16 hi + lo pairs: over inputs that fill
+    the spectra's range (0 and 255 only, one channel with a full-scale tone) or
+    hardly use it (127 and 128 only, a single sample away from the zero level)
+    its error stays what float32 transforms alone may make: one rounding of
+    2^-24 per stage of the two transforms, 2 log2(nfft) stages."""
+    rng = np.random.default_rng(nfft + nbits + len(kind))
+    nch, nsamps = 48, nfft + nfft // 8 + 77
+    dt, f0, df = 64e-6, 1581.8, -2.0
+    top = (1 << nbits) - 1
+    if kind == "saturated":
+        s = rng.integers(0, 2, size=(nsamps, nch)) * 255
+    elif kind == "faint":
+        s = rng.integers(127, 129, size=(nsamps, nch))
+    elif kind == "impulse":
+        s = np.full((nsamps, nch), 128)
+        s[nsamps // 3, nch // 2] = 255
+    else:
+        s = np.clip(np.rint(rng.normal(0.5 * top + 0.5, 0.16 * top + 0.3, size=(nsamps, nch))), 0, top)
+        if kind == "tone":
+            s[:, 5] = 255 * (np.arange(nsamps) // 4 % 2)
+    s = s.astype(np.uint8)
+    dms = np.linspace(0, 110, 20, dtype=f32)
+    plan = _fdd_plan(dd, nch, dt, f0, df, nfft=nfft, prec=dd.FDD_FP32)
+    plan.set_dm_list(dms)
+    out = plan.execute(dd.pack_samples(s, nbits), nbits, 32)
+    delays = orc.delay_table(nch, f32(dt), f32(f0), f32(df))
+    ref = orc.fdd_timeseries(nch, delays, dms, nsamps, plan.max_delay, s, nbits=nbits)
+    assert rel_l2(out, ref) < 2 * np.log2(nfft) * 2.0**-24
+    plan.close()
+
+
 def test_fdd_valu_and_mfma_fp32_agree(dd, orc, monkeypatch):
     rng = np.random.default_rng(12)
     nch, nsamps = 96, 40000
