@@ -106,6 +106,12 @@ constexpr size_t kYBudget = size_t(24) << 30;
 // Memory the channel spectra of one group of beams may take (batched beams).
 constexpr size_t kZBudget = size_t(32) << 30;
 
+// Measured costs the segment length is chosen by (ns; 1024 ch x 2^20 samples):
+// the contraction of one tile of 8 chunks per bin, DM and channel, and the
+// transforms per sample of a chunk (on chip, and split beyond 65536).
+constexpr double kPhasorTiles = 1.3, kTile = 1.33e-4;
+constexpr double kTransform = 2.3e-3, kSplitTransform = 4.3e-3;
+
 bool env_flag(const char* name)
 {
     const char* s = std::getenv(name);
@@ -362,38 +368,51 @@ void FDDGPUPlan::prepare_tables()
 }
 
 // Overlap-save segment length for series with nsc[0..n) outputs per DM: the
-// requested one, else the supported length (2^13 .. 2^18) with the smallest
-// contraction volume (chunk columns of the contraction kernel's tiles, padding
-// included, times nfft/2 + 1). The reference instead
-// doubles nfft from 16384 until a fifth of it covers the maximum delay
-// (src/fdd/FDDGPUPlan.cpp:756-762); the smallest volume needs fewer complex
-// multiply-accumulates for the same outputs.
+// requested one, else the supported length (2^13 .. 2^18) with the least
+// estimated time. The reference instead doubles nfft from 16384 until a fifth
+// of it covers the maximum delay (src/fdd/FDDGPUPlan.cpp:756-762).
 size_t FDDGPUPlan::segment_length(const size_t* nsc, size_t n) const
 {
     const FDDState& st = *m_state;
     const size_t dmax = (size_t)st.dmax;
     size_t nfft = st.nfft_req;
     if (!nfft) {
-        // smallest contraction volume (chunk columns the kernel computes,
-        // padding included) x (nfft/2 + 1) among the supported lengths
+        // Contraction: a chunk group of ntl 8-chunk tiles costs ntl tiles of
+        // products plus the phasors, kPhasorTiles tiles' worth whatever its
+        // width (1024 ch x 2048 DMs x 65536: one tile 20.9 ms, three 38.5 ms),
+        // for every bin, channel and DM, the DMs in whole waves of 32.
+        // Transforms: one per chunk and channel, one per chunk and DM.
+        // The smallest volume of columns x bins, which this replaces, left out
+        // phasors and transforms and took 131072 and one tile of 5 chunks at
+        // 1024 ch x 2^19 x 1000 DMs in float32 (29.6 ms) where 65536 and two
+        // tiles of 11 take 18.3 ms, and at 8 beams x 15625 x 3000 DMs in
+        // bfloat16 65536 (36.4 ms) instead of 32768 (27.1 ms). The float16
+        // form keeps the smallest volume: its rounding (2e-4 of the result)
+        // depends on the segment length, and an output should not.
         const Contraction kind = contraction_kind(st);
-        size_t best = ~size_t(0);
+        const double dms = (double)round_up(std::max<size_t>(m_dm_count, 1), 32);
+        double best = -1;
         for (size_t cand = 8192; cand <= 262144; cand *= 2) {
             if (cand < dmax + 2 + 2) continue;
             const size_t good = (cand - dmax) & ~size_t(1);
             size_t chunks = 0;
             for (size_t i = 0; i < n; ++i) chunks += div_up(nsc[i], good);
-            size_t cols = chunks;
+            double columns = (double)chunks, tiles = columns / 8;  // computed chunk columns, padding included
             if (kind == Contraction::MFMA32) {
-                cols = round_up(chunks, 32);
+                columns = (double)round_up(chunks, 32);
+                tiles = columns / 8;
             } else if (kind == Contraction::MFMA16) {
                 int ntl = 1;
                 size_t groups = 0;
                 dd_fdd_mfma16_tiles(chunks, (int)st.precision, &ntl, &groups);
-                cols = groups * (size_t)ntl * 8;
+                columns = (double)(groups * (size_t)ntl * 8);
+                tiles = (double)groups * ((double)ntl + kPhasorTiles);
             }
-            const size_t cost = cols * (cand / 2 + 1);
-            if (cost < best) { best = cost; nfft = cand; }
+            double cost = kTile * tiles * (double)(cand / 2 + 1) * dms * (double)padded_channels(m_nchans) +
+                          (cand > 65536 ? kSplitTransform : kTransform) * (double)chunks * (double)cand *
+                              (dms + (double)m_nchans);
+            if (st.precision == DEDISP_AMD_FDD_FP16) cost = columns * (double)(cand / 2 + 1);
+            if (best < 0 || cost < best) best = cost, nfft = cand;
         }
         if (!nfft) DD_THROW(DEDISP_UNKNOWN_ERROR);  // max delay beyond the largest segment
     }

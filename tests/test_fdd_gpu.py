@@ -495,3 +495,21 @@ def test_fdd_long_delay_batch_split_segments(dd, orc, nfft):
         ref = orc.fdd_timeseries(g["nch"], delays, dms, b.shape[0], plan.max_delay, b)
         assert rel_l2(o, ref) < PREC_TOL["bf16"]
     plan.close()
+
+
+@pytest.mark.parametrize("prec", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("ndm", [1, 31, 32, 33, 224, 225, 256, 257, 289])
+def test_fdd_waves_past_the_last_dm(dd, orc, prec, ndm):
+    """DM counts that leave waves of the contraction's last block without a DM."""
+    nch, nsamps, dt, f0, df = 72, 21001, 64e-6, 1581.8, -1.0
+    dms = np.linspace(0, 40, ndm, dtype=f32)
+    p = {"fp32": dd.FDD_FP32, "bf16": dd.FDD_BF16, "fp16": dd.FDD_FP16}[prec]
+    plan = _fdd_plan(dd, nch, dt, f0, df, nfft=8192, prec=p)
+    plan.set_dm_list(dms)
+    data = np.random.default_rng(ndm).integers(0, 256, size=(nsamps, nch)).astype(np.uint8)
+    out = plan.execute(data, 8, 32)
+    delays = orc.delay_table(nch, f32(dt), f32(f0), f32(df))
+    ref = orc.fdd_timeseries(nch, delays, dms, nsamps, plan.max_delay, data)
+    assert rel_l2(out, ref) < PREC_TOL[prec]
+    assert rel_l2(out[-1], ref[-1]) < PREC_TOL[prec]
+    plan.close()
