@@ -1165,52 +1165,62 @@ __global__ __launch_bounds__(256) void fourier_step_c_k(const float2* __restrict
     out[row * out_stride + k] = make_float2(e.x + r.x, e.y + r.y);
 }
 
-// Steps B and C in one pass for even m <= 144. A tile is columns A = 64w + l
-// and their mirrors B = 8192 - A (l < 64, all m rows) of one row: the
-// workgroup stages them in LDS, and each of its BC_WAVES waves sums BC_KH of the
-// radix-2 outputs k (E[k] / O[k] over the even / odd rows, as step B) for
-// column A and, at h-1-k, for column B, then pairs them. The real-input
-// pairing of bin kk = k2 + 8192 k1 takes Z[L - kk], which for k2 = A >= 1 is
-// row m-1-k1 of column B: rows k and k+h of A pair with rows 2h-1-k and h-1-k
-// of B, and the other way round. Column 4096 is its own mirror (B = A; its B
-// outputs are not written again); column 0 is paired within itself by
-// fourier_col0_k. Each column is read from HBM once, and the intermediate Z
-// never goes to HBM. The grid is persistent (tiles t = blockIdx.x + i
-// gridDim.x, w = t % 65, row = t / 65): the next tile's loads are in flight
-// in registers while the current one is summed.
-// Two shapes: BC_MAXM = 72 with 5 outputs per wave (LDS of two workgroups
-// per CU) and 144 with 9 (one workgroup per CU).
-constexpr int BC_WAVES = 8;
-constexpr int BC_NT = BC_WAVES * 64;
+// Steps B and C in one pass for m <= 144. A tile is columns A = 64w + l and
+// their mirrors B = 8192 - A (l < 64, all m rows) of one row: the workgroup
+// stages them in LDS, its waves sum the m-point transforms of both, write them
+// back to the tile and pair them. The real-input pairing of bin kk = k2 + 8192
+// k1 takes Z[L - kk], which for k2 >= 1 is row m-1-k1 of the mirror column.
+// Column 4096 is its own mirror (its B outputs are not written again); column
+// 0 is paired within itself by fourier_col0_k. Each column is read from HBM
+// once, and the intermediate Z never goes to HBM. The grid is persistent
+// (tiles t = blockIdx.x + i gridDim.x, w = t % 65, row = t / 65): the next
+// tile's loads are in flight in registers while the current one is summed.
+//
+// The m-point sums fold the rows in pairs: with u_p = a_p + a_{m-p} and
+// v_p = a_p - a_{m-p},
+//   X[k], X[m-k] = C[k] -+ i S[k],  C[k] = a_0 (+ (-1)^k a_{m/2}) + sum_p u_p cos(2 pi p k/m),
+//                                   S[k] = sum_p v_p sin(2 pi p k/m),  0 < p < m/2,
+// four multiply-adds for two outputs of two inputs, for odd and even m alike,
+// where sums over even and odd rows take eight and even m only. A wave takes
+// BC_KH of the floor(m/2)+1 values k for both columns. The shape is the
+// smallest tile that holds m rows, with the registers capped for as many
+// workgroups per CU (PER_CU) as its LDS allows, so that one's loads and
+// barriers pass beside another's sums. 1024 rows of m = 33: 1.13 ms (4.4 GB
+// read and written, 0.95 ms at the copy rate), where fourier_step_b_k, which
+// reads a column ceil(m/16) times, and fourier_step_c_k took 4.88 + 1.03 ms;
+// 512 rows of even m = 8, 16, 66, 144: 129, 377, 1365, 5007 us, with separate
+// even and odd sums and one of two tiles (72 or 144 rows) 335, 440, 1559, 6523.
 constexpr int BC_TILES_PER_ROW = 65;
 
-template <int BC_MAXM, int BC_KH>
-__global__ __launch_bounds__(BC_NT) void fourier_step_bc_k(const float2* __restrict__ A, size_t a_stride,
-                                                         size_t m, uint32_t nrows,
+template <int BC_MAXM, int BC_KH, int WAVES, int PER_CU>
+__global__ __launch_bounds__(WAVES * 64, WAVES * PER_CU / 4) void fourier_step_bc_k(const float2* __restrict__ A, size_t a_stride,
+                                                         size_t m_, uint32_t nrows,
                                                          const float2* __restrict__ twL,
                                                          const float2* __restrict__ twN, float2* __restrict__ out,
                                                          size_t out_stride)
 {
-    constexpr int BC_RPT = BC_MAXM * 128 / BC_NT;              // staged values per thread
+    constexpr int NT = WAVES * 64;
+    constexpr int BC_RPT = BC_MAXM * 128 / NT;              // staged values per thread
     constexpr int BC_LDS = 2 * BC_MAXM + BC_MAXM * 128;        // float2: W_m^e, W_N^{8192 k1}, [row][128] values
-    static_assert(BC_MAXM / 2 <= BC_WAVES * BC_KH && BC_NT % 128 == 0 && BC_MAXM % (BC_NT / 128) == 0,
-                  "the waves cover h = m/2 outputs, the threads the staged rows");
+    static_assert(NT % 128 == 0 && BC_MAXM % (NT / 128) == 0, "the threads cover the staged rows");
     __shared__ float2 bc_lds[BC_LDS];
     float2* const wt = bc_lds;                   // W_m^e, e < m
     float2* const wk = bc_lds + BC_MAXM;         // W_N^{8192 k1}, k1 < m
     float2* const col = bc_lds + 2 * BC_MAXM;    // [row][128]: lane l's column A at l, B at 64 + l
-    const uint32_t h = (uint32_t)(m / 2);
+    const uint32_t m = (uint32_t)m_;
+    const uint32_t npair = (m - 1) / 2;          // row pairs (p, m-p)
+    const uint32_t nk = m / 2 + 1;               // values k summed (X[k] and X[m-k])
     const int t = threadIdx.x, lane = t & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const uint32_t kb = wave * BC_KH;
     const uint32_t ntile = BC_TILES_PER_ROW * nrows;
-    for (uint32_t i = t; i < m; i += BC_NT) wt[i] = twL[(size_t)i * 8192], wk[i] = twN[(size_t)i * 8192];
+    for (uint32_t i = t; i < m; i += NT) wt[i] = twL[(size_t)i * 8192], wk[i] = twN[(size_t)i * 8192];
     // staging: thread t holds tile column c = t & 127 at rows RS i + (t >> 7)
-    // (RS = BC_NT / 128 rows a step), i < BC_RPT, the rows past m - 1 clamped
+    // (RS = NT / 128 rows a step), i < BC_RPT, the rows past m - 1 clamped
     // to m - 1 (loaded and stored, never summed); columns clamped into
     // [1, 4096] (the lanes past them compute but do not write). Byte offsets
     // from the row base fit 32 bits (< BC_MAXM x 8192 x 8 <= 144 x 8192 x 8)
-    constexpr uint32_t RS = BC_NT / 128;
+    constexpr uint32_t RS = NT / 128;
     const uint32_t sc = t & 127, sr0 = t >> 7;
     float2 v[BC_RPT];
     auto load = [&](uint32_t tile) {
@@ -1220,7 +1230,7 @@ __global__ __launch_bounds__(BC_NT) void fourier_step_bc_k(const float2* __restr
         const uint32_t off0 = ((sc < 64) ? ca : 8192 - ca) * 8;
         // opaque copy of the last row: keeps the clamped offsets from being
         // hoisted out of the tile loop into as many scalar registers
-        uint32_t rlast = 2 * h - 1;
+        uint32_t rlast = m - 1;
         asm volatile("" : "+s"(rlast));
 #pragma unroll
         for (int i = 0; i < BC_RPT; ++i) {
@@ -1228,80 +1238,96 @@ __global__ __launch_bounds__(BC_NT) void fourier_step_bc_k(const float2* __restr
             v[i] = *reinterpret_cast<const float2*>(base + off0 + r * (8192 * 8));
         }
     };
-    // pairing of bin kk = k2 + 8192 k1 with Z[L - kk] (the step-C formula);
-    // W_N^kk = W_N^{k2} W_N^{8192 k1}: the lane's column factor times an LDS
-    // entry (two exact table values) rather than a gather from the L-entry
-    // table per output
-    auto pair_out = [&](float2* o_row, uint32_t k2, uint32_t k1, float2 wc, float2 za, float2 zb) {
-        const float2 ev = make_float2(0.5f * (za.x + zb.x), 0.5f * (za.y - zb.y));
-        const float2 d = make_float2(za.x - zb.x, za.y + zb.y);
-        const float2 o = make_float2(0.5f * d.y, -0.5f * d.x);
-        const float2 r = cmul(o, cmul(wc, wk[k1]));
-        o_row[k2 + 8192 * (size_t)k1] = make_float2(ev.x + r.x, ev.y + r.y);
-    };
     uint32_t tile = blockIdx.x;
     if (tile < ntile) load(tile);
     for (; tile < ntile; tile += gridDim.x) {
-        __syncthreads();  // the previous tile's sums have read col (and wt is written)
+        __syncthreads();  // the previous tile's pairing has read col (and wt is written)
 #pragma unroll
         for (int i = 0; i < BC_RPT; ++i) col[(RS * i + sr0) * 128 + sc] = v[i];
         __syncthreads();
         if (tile + gridDim.x < ntile) load(tile + gridDim.x);
-        if (kb < h) {
-            // all BC_KH outputs are summed (the ones past h - 1 are not written):
-            // no branch in the loop, and e stays in scalar registers
-            float2 EA[BC_KH], OA[BC_KH], EB[BC_KH], OB[BC_KH];
-            uint32_t e[BC_KH + 1];  // (p * (kb + j)) mod h, j <= BC_KH
+        float2 CA[BC_KH], SA[BC_KH], CB[BC_KH], SB[BC_KH];
+        if (kb < nk) {
+            // all BC_KH values are summed (the ones past nk - 1 repeat it and
+            // are not written): no branch in the loop, and e stays in scalar
+            // registers
+            uint32_t e[BC_KH], ks[BC_KH];  // (p * k) mod m, k
+            const float2 a0 = col[lane], b0 = col[64 + lane];
+            float2 ah = make_float2(0.f, 0.f), bh = ah;
+            if (m % 2 == 0) ah = col[(m / 2) * 128 + lane], bh = col[(m / 2) * 128 + 64 + lane];
 #pragma unroll
-            for (int j = 0; j < BC_KH; ++j) EA[j] = OA[j] = EB[j] = OB[j] = make_float2(0.f, 0.f);
-#pragma unroll
-            for (int j = 0; j <= BC_KH; ++j) e[j] = 0;
-            for (uint32_t p = 0; p < h; ++p) {
-                const float2 ae = col[(2 * p) * 128 + lane], ao = col[(2 * p + 1) * 128 + lane];
-                const float2 be = col[(2 * p) * 128 + 64 + lane], bo = col[(2 * p + 1) * 128 + 64 + lane];
+            for (int j = 0; j < BC_KH; ++j) {
+                ks[j] = min(kb + j, nk - 1);
+                e[j] = ks[j];
+                const float sg = (ks[j] & 1u) ? -1.f : 1.f;
+                CA[j] = make_float2(fmaf(sg, ah.x, a0.x), fmaf(sg, ah.y, a0.y));
+                CB[j] = make_float2(fmaf(sg, bh.x, b0.x), fmaf(sg, bh.y, b0.y));
+                SA[j] = SB[j] = make_float2(0.f, 0.f);
+            }
+#pragma unroll 1
+            for (uint32_t p = 1; p <= npair; ++p) {
+                const float2 a1 = col[p * 128 + lane], a2 = col[(m - p) * 128 + lane];
+                const float2 b1 = col[p * 128 + 64 + lane], b2 = col[(m - p) * 128 + 64 + lane];
+                const float2 ua = cadd(a1, a2), va = csub(a1, a2), ub = cadd(b1, b2), vb = csub(b1, b2);
 #pragma unroll
                 for (int j = 0; j < BC_KH; ++j) {
-                    // A at k = kb + j: W_h^{p k}; B at h-1-k: W_h^{p (h-1-k)} = conj W_h^{p (k+1)}
-                    const float2 wa = wt[2 * e[j]], wb0 = wt[2 * e[j + 1]];
-                    const float2 wb = make_float2(wb0.x, -wb0.y);
-                    EA[j].x = fmaf(ae.x, wa.x, fmaf(-ae.y, wa.y, EA[j].x));
-                    EA[j].y = fmaf(ae.x, wa.y, fmaf(ae.y, wa.x, EA[j].y));
-                    OA[j].x = fmaf(ao.x, wa.x, fmaf(-ao.y, wa.y, OA[j].x));
-                    OA[j].y = fmaf(ao.x, wa.y, fmaf(ao.y, wa.x, OA[j].y));
-                    EB[j].x = fmaf(be.x, wb.x, fmaf(-be.y, wb.y, EB[j].x));
-                    EB[j].y = fmaf(be.x, wb.y, fmaf(be.y, wb.x, EB[j].y));
-                    OB[j].x = fmaf(bo.x, wb.x, fmaf(-bo.y, wb.y, OB[j].x));
-                    OB[j].y = fmaf(bo.x, wb.y, fmaf(bo.y, wb.x, OB[j].y));
+                    const float2 w = wt[e[j]];  // (cos, -sin)
+                    CA[j].x = fmaf(ua.x, w.x, CA[j].x);
+                    CA[j].y = fmaf(ua.y, w.x, CA[j].y);
+                    SA[j].x = fmaf(va.x, w.y, SA[j].x);
+                    SA[j].y = fmaf(va.y, w.y, SA[j].y);
+                    CB[j].x = fmaf(ub.x, w.x, CB[j].x);
+                    CB[j].y = fmaf(ub.y, w.x, CB[j].y);
+                    SB[j].x = fmaf(vb.x, w.y, SB[j].x);
+                    SB[j].y = fmaf(vb.y, w.y, SB[j].y);
                 }
 #pragma unroll
-                for (int j = 0; j <= BC_KH; ++j) {
-                    // x mod h for x < 2h as a minimum (x - h wraps when x < h):
+                for (int j = 0; j < BC_KH; ++j) {
+                    // x mod m for x < 2m as a minimum (x - m wraps when x < m):
                     // selects in scalar registers, where a compare-and-subtract
                     // was lowered to vector instructions
-                    const uint32_t x = e[j] + kb + j;
-                    e[j] = min(x, x - h);
+                    const uint32_t x = e[j] + ks[j];
+                    e[j] = min(x, x - m);
                 }
             }
-            const uint32_t w = tile % BC_TILES_PER_ROW, row = tile / BC_TILES_PER_ROW;
-            const uint32_t cA = 64 * w + lane, cB = 8192 - cA;
-            if (cA >= 1 && cA <= 4096) {
-                float2* o_row = out + row * out_stride;
-                const float2 wA = twN[cA], wB = twN[cB];
+        }
+        __syncthreads();  // every wave has read the staged rows
+        if (kb < nk) {
 #pragma unroll
-                for (int j = 0; j < BC_KH; ++j) {
-                    const uint32_t k = kb + j;
-                    if (k < h) {
-                        const uint32_t kB = h - 1 - k;
-                        const float2 ta = cmul(OA[j], wt[k]), tb = cmul(OB[j], wt[kB]);
-                        const float2 zA0 = cadd(EA[j], ta), zA1 = csub(EA[j], ta);  // rows k, k+h of A
-                        const float2 zB0 = cadd(EB[j], tb), zB1 = csub(EB[j], tb);  // rows h-1-k, 2h-1-k of B
-                        pair_out(o_row, cA, k, wA, zA0, zB1);
-                        pair_out(o_row, cA, k + h, wA, zA1, zB0);
-                        if (cA < 4096) {
-                            pair_out(o_row, cB, kB, wB, zB0, zA1);
-                            pair_out(o_row, cB, kB + h, wB, zB1, zA0);
-                        }
+            for (int j = 0; j < BC_KH; ++j) {
+                const uint32_t k = kb + j;
+                if (k < nk) {
+                    // S holds -sum v sin: X[k] = C + i S, X[m-k] = C - i S
+                    col[k * 128 + lane] = make_float2(CA[j].x - SA[j].y, CA[j].y + SA[j].x);
+                    col[k * 128 + 64 + lane] = make_float2(CB[j].x - SB[j].y, CB[j].y + SB[j].x);
+                    if (k > 0 && 2 * k < m) {
+                        col[(m - k) * 128 + lane] = make_float2(CA[j].x + SA[j].y, CA[j].y - SA[j].x);
+                        col[(m - k) * 128 + 64 + lane] = make_float2(CB[j].x + SB[j].y, CB[j].y - SB[j].x);
                     }
+                }
+            }
+        }
+        __syncthreads();
+        // pairing of bin kk = k2 + 8192 k1 with Z[L - kk] (the step-C formula);
+        // W_N^kk = W_N^{k2} W_N^{8192 k1}: the column's factor times an LDS
+        // entry (two exact table values) rather than a gather from the L-entry
+        // table per output
+        const uint32_t w = tile % BC_TILES_PER_ROW, row = tile / BC_TILES_PER_ROW;
+        const uint32_t cA = 64 * w + (sc & 63);
+        if (cA >= 1 && (cA < 4096 || (cA == 4096 && sc < 64))) {
+            const uint32_t k2 = (sc < 64) ? cA : 8192 - cA;
+            const float2 wc = twN[k2];
+            float2* o_row = out + row * out_stride + k2;
+#pragma unroll 2
+            for (int i = 0; i < BC_RPT; ++i) {
+                const uint32_t k1 = RS * i + sr0;
+                if (k1 < m) {
+                    const float2 za = col[k1 * 128 + sc], zb = col[(m - 1 - k1) * 128 + (sc ^ 64)];
+                    const float2 ev = make_float2(0.5f * (za.x + zb.x), 0.5f * (za.y - zb.y));
+                    const float2 d = make_float2(za.x - zb.x, za.y + zb.y);
+                    const float2 o = make_float2(0.5f * d.y, -0.5f * d.x);
+                    const float2 r = cmul(o, cmul(wc, wk[k1]));
+                    o_row[8192 * (size_t)k1] = make_float2(ev.x + r.x, ev.y + r.y);
                 }
             }
         }
@@ -1348,15 +1374,15 @@ __global__ __launch_bounds__(256) void fourier_col0_k(const float2* __restrict__
 
 }  // namespace
 
-// Whether steps B and C run fused: even m <= 144, whose h = m/2 outputs the
-// waves of fourier_step_bc_k cover (DEDISP_FDD_BC=0 keeps the two passes).
+// Whether steps B and C run fused: m <= 144, whose rows an LDS tile holds
+// (DEDISP_FDD_BC=0 keeps the two passes).
 inline bool bc_fused(size_t m)
 {
     static const bool off = [] {
         const char* v = std::getenv("DEDISP_FDD_BC");
         return v && v[0] == '0';
     }();
-    return !off && m % 2 == 0 && m <= 144;
+    return !off && m <= 144;
 }
 
 extern "C" hipError_t dd_fdd_rfft_rows(const float* S, size_t s_stride, size_t nrows, size_t N,
@@ -1387,21 +1413,25 @@ extern "C" hipError_t dd_fdd_rfft_rows(const float* S, size_t s_stride, size_t n
         if (e != hipSuccess) return e;
         if (bc_fused(m)) {
             // steps B and C in one pass (column 0 on its own)
-            // persistent: two workgroups per CU for m <= 72 (the LDS tile
-            // allows two), one for m <= 144
+            // persistent: as many workgroups per CU as the LDS tile of the
+            // smallest shape that holds the m rows (and m / 2 + 1 values k) allows
             int dev = 0, ncu = 0;
             e = hipGetDevice(&dev);
             if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
             if (e != hipSuccess) return e;
             const size_t ntile = (size_t)BC_TILES_PER_ROW * nr;
-            const bool small = m <= 72;
-            const unsigned grid = (unsigned)std::min<size_t>(ntile, (small ? 2 : 1) * (size_t)std::max(ncu, 1));
-            if (small)
-                hipLaunchKernelGGL((fourier_step_bc_k<72, 5>), dim3(grid), dim3(BC_NT), 0, stream, Sr, sp, m,
-                                   (uint32_t)nr, twL, twN, out + r0 * out_stride, out_stride);
-            else
-                hipLaunchKernelGGL((fourier_step_bc_k<144, 9>), dim3(grid), dim3(BC_NT), 0, stream, Sr, sp, m,
-                                   (uint32_t)nr, twL, twN, out + r0 * out_stride, out_stride);
+#define DD_BC(MAXM, KH, WAVES, PER_CU)                                                                          \
+    do {                                                                                                        \
+        const unsigned grid = (unsigned)std::min<size_t>(ntile, (PER_CU) * (size_t)std::max(ncu, 1));            \
+        hipLaunchKernelGGL((fourier_step_bc_k<MAXM, KH, WAVES, PER_CU>), dim3(grid), dim3((WAVES) * 64), 0,      \
+                           stream, Sr, sp, m, (uint32_t)nr, twL, twN, out + r0 * out_stride, out_stride);        \
+    } while (0)
+            if (m < 16) DD_BC(16, 1, 8, 4);
+            else if (m < 48) DD_BC(48, 3, 8, 3);
+            else if (m < 64) DD_BC(64, 4, 8, 2);
+            else if (m <= 72) DD_BC(72, 5, 8, 2);
+            else DD_BC(144, 5, 16, 1);
+#undef DD_BC
             e = hipGetLastError();
             if (e != hipSuccess) return e;
             hipLaunchKernelGGL(fourier_col0_k, dim3(nr), dim3(256), 0, stream, Sr, sp, m, twL, twN,

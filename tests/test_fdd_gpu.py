@@ -497,6 +497,26 @@ def test_fdd_long_delay_batch_split_segments(dd, orc, nfft):
     plan.close()
 
 
+@pytest.mark.parametrize("m", [1, 2, 3, 5, 14, 15, 16, 17, 46, 47, 48, 49, 62, 63, 64, 65, 72, 73, 143, 144, 145])
+def test_fdd_fourier_row_counts(dd, orc, m):
+    """The m-point step of the row transforms (N = 16384 m) at the edges of its
+    shapes and past the largest. One rounding of 2^-24 per stage of the chunk
+    transforms (two of at most 2^18) and of the 8192-point step, sqrt(m) for
+    the direct sums, and four for the twiddles and the pairing."""
+    nch, dt, f0, df = 8, 64e-6, 1581.8, -0.390625
+    dms = np.array([0, 3.3, 20], dtype=f32)
+    plan = dd.Plan(nch, dt, f0, df, impl=dd.FDD)
+    plan.set_dm_list(dms)
+    nsamps = 16384 * m - plan.max_delay - 5
+    assert plan.out_length(nsamps) == 16384 * m
+    data = np.random.default_rng(m).integers(0, 256, size=(nsamps, nch)).astype(np.uint8)
+    out = plan.execute(data, 8, 32)
+    delays = orc.delay_table(nch, f32(dt), f32(f0), f32(df))
+    ref = orc.fdd_fourier(nch, delays, dms, nsamps, plan.max_delay, data)
+    assert rel_l2(out, ref) < (2 * 18 + 13 + np.sqrt(m) + 4) * 2.0**-24
+    plan.close()
+
+
 @pytest.mark.parametrize("prec", ["fp32", "bf16", "fp16"])
 @pytest.mark.parametrize("ndm", [1, 31, 32, 33, 224, 225, 256, 257, 289])
 def test_fdd_waves_past_the_last_dm(dd, orc, prec, ndm):
