@@ -9,6 +9,7 @@
 #include <cstdint>
 #include <functional>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "dedisp.hpp"
@@ -32,6 +33,7 @@ struct DeviceBuffer {
     ~DeviceBuffer();
     void reserve(size_t n);   // ensures at least n bytes (contents not kept)
     void release();
+    void swap(DeviceBuffer& o) { std::swap(ptr, o.ptr), std::swap(bytes, o.bytes); }
     template <typename T> T* as() const { return static_cast<T*>(ptr); }
 };
 

@@ -111,6 +111,33 @@ hipError_t dd_tdd_dedisperse_lds_batch(const dd_tdd_beam* beams, const uint32_t*
                                        size_t ndm, dd_tdd_epilogue ep, dd_tdd_tiling tiling,
                                        hipStream_t stream);
 
+// Bit-plane channel sum (tdd_planes.hip): 1- to 8-bit input, the tilings with
+// samples_per_lane 64 (32 time runs x 2 positions per lane; chunk_channels
+// from dd_tdd_planes_chunk, 0 where no instantiation holds the sums; nchunk,
+// the channels over chunk_channels, rounded up to even). Rows come
+// from dd_tdd_transpose_planes: word (q*T + p)*nbits + b of a channel holds bit
+// b of samples q*32T + r*T + p at bit r (zero beyond nsamps); row_words is a
+// multiple of T*nbits. Per DM block: wstart [nchunk*chunk_channels][2] smallest
+// delay and number of each channel (past the last one, any of them), chunks [nchunk] positions staged per channel (a
+// multiple of 64, at most window_words, the LDS positions of a channel); code
+// [DM group][nchunk][DMs per wave][chunk_channels] LDS byte offsets of each
+// DM's window, (slot*window_words + delay - wstart) * nbits * 4, and for the
+// channels past the last one chunk_channels*window_words*nbits*4. Three tiles
+// are read from that of a window's start on: rows hold ntiles + (largest
+// wstart)/32T + 2 tiles.
+#define DD_TDD_PLANES_T 128
+#define DD_TDD_PLANES_SPL 64
+static inline int dd_tdd_tiling_is_planes(dd_tdd_tiling t) { return t.samples_per_lane == DD_TDD_PLANES_SPL; }
+unsigned dd_tdd_planes_chunk(unsigned nbits, size_t nact, unsigned dms_per_wave, unsigned waves);
+int dd_tdd_planes_tilings(unsigned nbits, dd_tdd_tiling* out, int max);
+hipError_t dd_tdd_transpose_planes(const uint8_t* in, size_t nsamps, size_t in_stride, unsigned nbits, size_t nchans,
+                                   uint32_t* out, size_t row_words, hipStream_t stream);
+hipError_t dd_tdd_dedisperse_planes(const uint32_t* rows, size_t row_words, unsigned nbits, const uint32_t* code,
+                                    const uint32_t* wstart, const uint32_t* chunks, unsigned nchunk, size_t nact,
+                                    size_t ndm, size_t nsamps_out, uint8_t* out, size_t out_stride,
+                                    dd_tdd_epilogue ep, dd_tdd_tiling tiling, const dd_tdd_beam* beams,
+                                    const uint32_t* tile_beam, size_t batch_tiles, hipStream_t stream);
+
 // The runs-layout channel sum (see dd_tdd_tiling_is_runs).
 hipError_t dd_tdd_dedisperse_runs(const uint32_t* rows, size_t row_words, const uint32_t* code,
                                   const int32_t* chan, const uint32_t* wstart, const uint32_t* chunks,

@@ -656,6 +656,8 @@ extern "C" int dd_tdd_lds_tilings(unsigned nbits, dd_tdd_tiling* out, int max)
         if (n < max && out) out[n] = dd_tdd_tiling{DD_TDD_RUNS_SPL, 2, 8, 16, 0};
         ++n;
     }
+    // the bit-plane kernel (tdd_planes.hip)
+    n += dd_tdd_planes_tilings(nbits, (n < max && out) ? out + n : nullptr, max - n);
 #define DD_LIST(NB, GG, DPW, WAVES)                                        \
     if (nbits == NB) {                                                     \
         if (n < max && out) {                                              \
@@ -672,6 +674,7 @@ extern "C" int dd_tdd_lds_supported(unsigned nbits, dd_tdd_tiling tl)
 {
     if (dd_tdd_tiling_is_runs(nbits, tl))
         return (tl.dms_per_wave == 4 && tl.waves == 4) || (tl.dms_per_wave == 2 && tl.waves == 8);
+    if (dd_tdd_tiling_is_planes(tl)) return dd_tdd_planes_chunk(nbits, 1, tl.dms_per_wave, tl.waves) != 0;
     const unsigned spw = 32 / nbits;
     if (tl.samples_per_lane % spw) return 0;
     const unsigned G = tl.samples_per_lane / spw;
@@ -695,6 +698,9 @@ extern "C" hipError_t dd_tdd_dedisperse_lds(const uint32_t* rows, size_t row_wor
         return dd_tdd_dedisperse_runs(rows, row_words, code, chan, wstart, chunks, maxc, nact, ndm, nsamps_out,
                                       out, out_stride, ep, tl.dms_per_wave, tl.waves, nullptr, nullptr, 0,
                                       stream);
+    if (dd_tdd_tiling_is_planes(tl))
+        return dd_tdd_dedisperse_planes(rows, row_words, nbits, code, wstart, chunks, maxc, nact, ndm,
+                                        nsamps_out, out, out_stride, ep, tl, nullptr, nullptr, 0, stream);
     const unsigned spw = 32 / nbits;
     const unsigned G = tl.samples_per_lane / spw;
     const uint32_t maxv = (1u << nbits) - 1u;
@@ -727,6 +733,9 @@ extern "C" hipError_t dd_tdd_dedisperse_lds_batch(const dd_tdd_beam* beams, cons
     if (dd_tdd_tiling_is_runs(nbits, tl))
         return dd_tdd_dedisperse_runs(nullptr, 0, code, chan, wstart, chunks, maxc, nact, ndm, 0, nullptr, 0, ep,
                                       tl.dms_per_wave, tl.waves, beams, tile_beam, ntiles, stream);
+    if (dd_tdd_tiling_is_planes(tl))
+        return dd_tdd_dedisperse_planes(nullptr, 0, nbits, code, wstart, chunks, maxc, nact, ndm, 0, nullptr,
+                                        0, ep, tl, beams, tile_beam, ntiles, stream);
     const unsigned spw = 32 / nbits;
     const unsigned G = tl.samples_per_lane / spw;
     const uint32_t maxv = (1u << nbits) - 1u;

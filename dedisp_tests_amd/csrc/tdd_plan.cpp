@@ -11,6 +11,7 @@
 // output samples, each reading its max_delay samples of overlap again
 // (src/tdd/TDDPlan.cpp:225-263, 354-420).
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cstdlib>
 #include <cstring>
@@ -21,16 +22,14 @@
 
 namespace dedisp {
 
-struct TDDState {
-    // device buffers, grown on demand and kept between executes
-    DeviceBuffer d_in;      // staged input (host-pointer mode)
-    DeviceBuffer d_rows;    // channel-major packed rows
-    DeviceBuffer d_out;     // staged output (host-pointer mode)
+// Tables of one channel-sum kernel for a DM range: host copies, device buffers
+// and what is derived from them.
+struct TDDTables {
     DeviceBuffer d_code;    // fast path [DM group][nact][DMs per wave] LDS offset | shift; generic [ndm][nact] delay
     DeviceBuffer d_chan;    // [nact] channel index
     DeviceBuffer d_weight;  // [nact] killmask weight (generic path)
     DeviceBuffer d_wstart;  // [ndmblk][nact] staged window start (fast path)
-    DeviceBuffer d_chunks;  // [ndmblk][maxc] staging chunks (runs-layout kernel)
+    DeviceBuffer d_chunks;  // [ndmblk][maxc] staging chunks (runs-layout and bit-plane kernels)
 
     // host copies of the tables (what the device buffers above hold once
     // uploaded): fast path delay codes or generic [ndm][nact] delays, channel
@@ -44,22 +43,55 @@ struct TDDState {
     unsigned long version = ~0ul;
     unsigned nbits = 0;
     size_t first_dm = ~size_t(0), dm_count = 0;
+    dd_tdd_tiling tiling_key{};
 
     // derived from the tables
     bool fast = false;
     dd_tdd_tiling tiling{};
     size_t nact = 0;
+    size_t code_per_dm = 0, wstart_per_blk = 0;  // fast path: words of d_code per DM, of d_wstart per DM block
     size_t dmax = 0;        // largest delay (samples) over the DMs in use
     size_t max_wstart = 0;  // fast path
-    unsigned maxc = 0;      // runs-layout kernel: chunk entries per DM block (terminator included)
+    unsigned maxc = 0;      // chunk entries per DM block (runs layout: terminator included)
+
+    void swap(TDDTables& o)
+    {
+        d_code.swap(o.d_code), d_chan.swap(o.d_chan), d_weight.swap(o.d_weight);
+        d_wstart.swap(o.d_wstart), d_chunks.swap(o.d_chunks);
+        h_tab.swap(o.h_tab), h_wstart.swap(o.h_wstart), h_chunks.swap(o.h_chunks);
+        h_chan.swap(o.h_chan), h_weight.swap(o.h_weight);
+        std::swap(uploaded, o.uploaded), std::swap(table_uid, o.table_uid);
+        std::swap(version, o.version), std::swap(nbits, o.nbits);
+        std::swap(first_dm, o.first_dm), std::swap(dm_count, o.dm_count), std::swap(tiling_key, o.tiling_key);
+        std::swap(fast, o.fast), std::swap(tiling, o.tiling), std::swap(nact, o.nact);
+        std::swap(code_per_dm, o.code_per_dm), std::swap(wstart_per_blk, o.wstart_per_blk);
+        std::swap(dmax, o.dmax), std::swap(max_wstart, o.max_wstart), std::swap(maxc, o.maxc);
+    }
+};
+
+// The tables in use, and (spare) those of the other kind: bit-plane ones for
+// large launches, packed-lane or runs-layout ones for small (planes says which
+// are in use).
+struct TDDState : TDDTables {
+    TDDTables spare;
+    bool planes = false;
+
+    // device buffers, grown on demand and kept between executes
+    DeviceBuffer d_in;      // staged input (host-pointer mode)
+    DeviceBuffer d_rows;    // channel-major packed rows
+    DeviceBuffer d_out;     // staged output (host-pointer mode)
+
     size_t row_words = 0;
 
     // the caller chose the gulp size (set_gulp_size): execute in gulps of it
     bool gulp_explicit = false;
 
+    // tables version, width and series length whose bit-plane rows exceed the
+    // scratch of execute_noalloc (packed lanes are used there)
+    std::array<uint64_t, 3> noalloc_packed = {~uint64_t(0), 0, 0};
+
     // tilings chosen by the autotuner, per input width (waves == 0: none)
     dd_tdd_tiling tuned[33] = {};
-    dd_tdd_tiling tiling_key{};
 
     // batched execution (own buffers, so a cached graph's pointers stay valid
     // whatever single executes do in between)
@@ -103,7 +135,7 @@ namespace {
 // Default tiling per input width (words per lane x SPW samples, DMs per wave,
 // waves); the chunk size is fitted to the LDS budget below. Overridden by the
 // environment variable DEDISP_TDD_TILING="samples_per_lane,dms_per_wave,waves,chunk".
-dd_tdd_tiling default_tiling(unsigned nbits)
+dd_tdd_tiling packed_tiling(unsigned nbits)
 {
     dd_tdd_tiling t{};
     // Measured on MI355X (channel-sum kernel, 2^20 samples, 16-channel
@@ -132,12 +164,46 @@ dd_tdd_tiling default_tiling(unsigned nbits)
     return t;
 }
 
+// Bit planes (tdd_planes.hip) for every sub-byte width and, 1 DM per wave for
+// its 18 counter planes, 8-bit: 1-bit, 512 ch x 200003 x 501 DMs 1.07 -> 0.38
+// ms per execute; 2-bit, 512 ch x 4 beams x 1024 DMs 21.7 -> 8.4 ms; 4-bit,
+// 1024 ch x 2^20 x 1167 DMs 22.8 -> 14.8 ms (runs layout before); 8-bit, 1024
+// ch x 15625 x 3000 DMs 2.03 -> 1.58 ms.
+dd_tdd_tiling default_tiling(unsigned nbits)
+{
+    if (nbits == 1 || nbits == 2 || nbits == 4) return dd_tdd_tiling{DD_TDD_PLANES_SPL, 2, 8, 16, 0};
+    if (nbits == 8) return dd_tdd_tiling{DD_TDD_PLANES_SPL, 1, 8, 16, 0};
+    return packed_tiling(nbits);
+}
+
+// Whether ntiles time tiles x dm_count DMs are too few for the bit-plane
+// kernel, whose workgroups are larger (4096 outputs) and fewer: below about 96
+// of them the smaller ones of the other kernels keep more of the chip busy
+// (2-bit, 256 ch, 16 DMs a block: 48 workgroups 0.93 of the packed lanes'
+// speed, 112 1.34; 8-bit, 8 DMs a block and a gain of 1.2 at most: 384
+// workgroups, 1.5 a CU, 0.9, 1500 1.28).
+size_t planes_tiles(size_t nsc) { return div_up(nsc, size_t(32) * DD_TDD_PLANES_T); }
+bool too_few_for_planes(unsigned nbits, size_t ntiles, size_t dm_count)
+{
+    const dd_tdd_tiling t = default_tiling(nbits);
+    return ntiles * div_up(dm_count, (size_t)t.dms_per_wave * t.waves) < (nbits == 8 ? 448u : 96u);
+}
+
 constexpr size_t kLdsBudget = 64 * 1024;  // bytes of LDS per workgroup
+// LDS of a bit-plane workgroup: two per CU, or (1 DM per wave, sub-byte, for
+// windows that 2 DMs per wave would not fit into that) one. 512 ch x 100000 x
+// 1000 DMs, delays 80 samples apart from DM to DM at the last channel: 1-bit
+// 0.55 ms with 1 DM per wave, 0.69 with 2 in one workgroup per CU, 1.35 on
+// packed lanes; 4-bit 1.07, 1.31, 1.31. 8-bit with one workgroup per CU lost to
+// the packed lanes, 2.60 against 2.16 ms.
+constexpr size_t kPlanesLds = 80 * 1024, kPlanesLdsOne = 158 * 1024;
 
 // Output samples per time tile of the channel-sum kernel: 7 runs of 256 for
-// the runs-layout kernel, 64 lanes x samples_per_lane for the packed-lane one.
+// the runs-layout kernel, 32 for the bit-plane kernel, 64 lanes x
+// samples_per_lane for the packed-lane one.
 size_t tile_samples(unsigned nbits, const dd_tdd_tiling& t)
 {
+    if (dd_tdd_tiling_is_planes(t)) return size_t(32) * DD_TDD_PLANES_T;
     return dd_tdd_tiling_is_runs(nbits, t) ? size_t(7 * 256) : size_t(64) * t.samples_per_lane;
 }
 
@@ -221,6 +287,79 @@ bool build_runs_tables(const std::vector<uint32_t>& d, size_t dm_count, size_t n
     return true;
 }
 
+// Words per channel of the bit-plane rows for nsc outputs: whole tiles, and the
+// tiles a window reads past the last one (from its start's on, three).
+size_t planes_row_words(unsigned nbits, size_t nsc, size_t max_wstart)
+{
+    constexpr size_t T = DD_TDD_PLANES_T, tile = 32 * T;
+    return (div_up(nsc, tile) + max_wstart / tile + 2) * T * nbits;
+}
+
+// The rows of a series in the layout the tiling's kernel reads.
+hipError_t transpose_rows(bool planes, const uint8_t* in, size_t nsamps, size_t in_stride, unsigned nbits,
+                          size_t nchans, uint32_t* rows, size_t row_words, hipStream_t stream)
+{
+    return planes ? dd_tdd_transpose_planes(in, nsamps, in_stride, nbits, nchans, rows, row_words, stream)
+                  : dd_tdd_transpose(in, nsamps, in_stride, nbits, nchans, rows, row_words, stream);
+}
+
+// Tables of the bit-plane channel sum (tdd_planes.hip) from the integer delays
+// d[dm][j]; nact channels in an even number of chunks of tl.chunk_channels, the
+// last ones filled up with channels of zeros. False when a chunk's windows
+// exceed the LDS allowed or no instantiation holds the sums.
+bool build_planes_tables(const std::vector<uint32_t>& d, const std::vector<int32_t>& chan, size_t dm_count,
+                         unsigned nbits, dd_tdd_tiling& tl, std::vector<uint32_t>& code,
+                         std::vector<uint32_t>& wstart, std::vector<uint32_t>& chunks, unsigned& maxc,
+                         size_t& max_wstart)
+{
+    const size_t nact = chan.size();
+    const size_t CC = dd_tdd_planes_chunk(nbits, nact, tl.dms_per_wave, tl.waves);
+    if (CC == 0 || nact == 0 || dm_count == 0) return false;
+    const size_t DPW = tl.dms_per_wave, WAVES = tl.waves, DPB = DPW * WAVES;
+    const size_t nchunk = round_up(div_up(nact, CC), 2), ndmblk = div_up(dm_count, DPB);
+    wstart.assign(ndmblk * nchunk * CC * 2, 0);
+    chunks.assign(ndmblk * nchunk, DD_TDD_PLANES_T);
+    max_wstart = 0;
+    size_t stride = DD_TDD_PLANES_T;
+    for (size_t b = 0; b < ndmblk; ++b) {
+        const size_t i0 = b * DPB, i1 = std::min(dm_count, i0 + DPB);
+        for (size_t j = 0; j < nact; ++j) {
+            uint32_t lo = ~0u, hi = 0;
+            for (size_t i = i0; i < i1; ++i) {
+                lo = std::min(lo, d[i * nact + j]);
+                hi = std::max(hi, d[i * nact + j]);
+            }
+            wstart[(b * nchunk * CC + j) * 2] = lo;
+            wstart[(b * nchunk * CC + j) * 2 + 1] = (uint32_t)chan[j];
+            max_wstart = std::max<size_t>(max_wstart, lo);
+            uint32_t& P = chunks[b * nchunk + j / CC];
+            P = std::max<uint32_t>(P, (uint32_t)round_up(DD_TDD_PLANES_T + size_t(hi - lo), 64));
+            stride = std::max<size_t>(stride, P);
+        }
+    }
+    const size_t most = (DPW == 1 && nbits < 8) ? kPlanesLdsOne : kPlanesLds;
+    if ((CC * stride + DD_TDD_PLANES_T) * nbits * 4 > most) return false;
+    tl.chunk_channels = (unsigned)CC;
+    tl.window_words = (unsigned)stride;
+    maxc = (unsigned)nchunk;
+    // DMs past the end repeat the last one; channels past the last one read the
+    // zeros after the windows
+    const size_t ngroups = ndmblk * WAVES;
+    code.assign(ngroups * nchunk * DPW * CC, 0);
+    for (size_t g = 0; g < ngroups; ++g) {
+        const uint32_t* ws = wstart.data() + g / WAVES * nchunk * CC * 2;
+        uint32_t* c = code.data() + g * nchunk * DPW * CC;
+        for (size_t i = 0; i < DPW; ++i) {
+            const uint32_t* dd = d.data() + std::min(g * DPW + i, dm_count - 1) * nact;
+            for (size_t j = 0; j < nchunk * CC; ++j) {
+                const size_t off = (j < nact) ? (j % CC) * stride + (dd[j] - ws[2 * j]) : CC * stride;
+                c[(j / CC * DPW + i) * CC + j % CC] = (uint32_t)(off * nbits * 4);
+            }
+        }
+    }
+    return true;
+}
+
 }  // namespace
 
 TDDPlan::TDDPlan(size_type nchans, float_type dt, float_type f0, float_type df, int device_idx)
@@ -248,19 +387,24 @@ std::atomic<uint64_t> g_table_uid{0};
 // and delay codes. Built on the host and cached per DM list / killmask / width
 // / DM range / tiling (independent of the series length); with upload they are
 // also copied to the plan's device buffers.
-void TDDPlan::prepare_tables(unsigned nbits, dedisp_size first_dm_idx, dedisp_size dm_count, bool upload)
+void TDDPlan::prepare_tables(unsigned nbits, dedisp_size first_dm_idx, dedisp_size dm_count, bool upload,
+                             bool packed)
 {
     GPUContext& ctx = *m_ctx;
     TDDState& st = *m_state;
     hipStream_t stream = ctx.exec;
     const size_t spw = 32 / nbits;
-    dd_tdd_tiling want = default_tiling(nbits);
-    if (st.tuned[nbits].waves) want = st.tuned[nbits];
+    dd_tdd_tiling want = packed ? packed_tiling(nbits) : default_tiling(nbits);
+    if (st.tuned[nbits].waves && !(packed && dd_tdd_tiling_is_planes(st.tuned[nbits]))) want = st.tuned[nbits];
     if (const char* env = std::getenv("DEDISP_TDD_TILING")) {
         unsigned a, b, c, e;
         if (std::sscanf(env, "%u,%u,%u,%u", &a, &b, &c, &e) == 4) {
             want.samples_per_lane = a; want.dms_per_wave = b; want.waves = c; want.chunk_channels = e;
         }
+    }
+    if (st.planes != (dd_tdd_tiling_is_planes(want) != 0)) {
+        st.swap(st.spare);
+        st.planes = !st.planes;
     }
     if (st.version != m_tables_version || st.nbits != nbits || st.first_dm != first_dm_idx ||
         st.dm_count != dm_count || std::memcmp(&st.tiling_key, &want, sizeof want) != 0) {
@@ -293,6 +437,24 @@ void TDDPlan::prepare_tables(unsigned nbits, dedisp_size first_dm_idx, dedisp_si
         std::vector<uint32_t> code, wstart, chunks;
         size_t max_wstart = 0, W = 0;
         unsigned maxc = 0;
+        if (fast && dd_tdd_tiling_is_planes(tl)) {
+            auto build = [&] {
+                return build_planes_tables(d, chan, dm_count, nbits, tl, code, wstart, chunks, maxc, max_wstart);
+            };
+            bool built = build();
+            if (!built && tl.dms_per_wave == 2) {
+                tl.dms_per_wave = 1;
+                built = build();
+            }
+            if (!built) {
+                tl = packed_tiling(nbits);
+                code.clear();
+                wstart.clear();
+                chunks.clear();
+                maxc = 0;
+                max_wstart = 0;
+            }
+        }
         if (fast && dd_tdd_tiling_is_runs(nbits, tl)) {
             size_t ww = 0;
             if (build_runs_tables(d, dm_count, nact, tl, code, wstart, chunks, maxc, max_wstart, ww)) {
@@ -307,7 +469,7 @@ void TDDPlan::prepare_tables(unsigned nbits, dedisp_size first_dm_idx, dedisp_si
                 max_wstart = 0;
             }
         }
-        if (fast && !dd_tdd_tiling_is_runs(nbits, tl)) {
+        if (fast && !dd_tdd_tiling_is_runs(nbits, tl) && !dd_tdd_tiling_is_planes(tl)) {
             const size_t G = tl.samples_per_lane / spw;
             const size_t dpb = (size_t)tl.waves * tl.dms_per_wave;
             const size_t ndmblk = div_up(dm_count, dpb);
@@ -375,6 +537,11 @@ void TDDPlan::prepare_tables(unsigned nbits, dedisp_size first_dm_idx, dedisp_si
         st.fast = fast;
         st.tiling = tl;
         st.nact = nact;
+        st.code_per_dm = st.wstart_per_blk = nact;
+        if (fast && dd_tdd_tiling_is_planes(tl)) {
+            st.code_per_dm = (size_t)maxc * tl.chunk_channels;
+            st.wstart_per_blk = 2 * st.code_per_dm;
+        }
         st.dmax = dmax;
         st.max_wstart = max_wstart;
     }
@@ -415,6 +582,8 @@ size_t TDDPlan::row_words_for(unsigned nbits, size_t nsamps, size_t nsc) const
     const TDDState& st = *m_state;
     const size_t spw = 32 / nbits;
     size_t row_words;
+    if (st.fast && dd_tdd_tiling_is_planes(st.tiling))
+        return planes_row_words(nbits, nsc, st.max_wstart);
     if (st.fast) {
         const size_t tile_words = tile_samples(nbits, st.tiling) / spw;
         const size_t ntiles = div_up(nsc, tile_words * spw);
@@ -526,7 +695,8 @@ void TDDPlan::execute_span(size_type nsamps, const byte_type* in, size_type in_n
     hipStream_t stream = ctx.exec;
 
     const unsigned nbits = (unsigned)in_nbits;
-    prepare_tables(nbits, first_dm_idx, dm_count);
+    prepare_tables(nbits, first_dm_idx, dm_count, true,
+                   !m_state->tuned[nbits].waves && too_few_for_planes(nbits, planes_tiles(nsc), dm_count));
     st.row_words = row_words_for(nbits, nsamps, nsc);
 
     // ---- input ----
@@ -548,7 +718,7 @@ void TDDPlan::execute_span(size_type nsamps, const byte_type* in, size_type in_n
     // ---- transpose ----
     st.d_rows.reserve(m_nchans * st.row_words * 4);
     ctx.timer.begin(StageTimer::UNPACK, stream);
-    DD_HIP(dd_tdd_transpose(d_in, nsamps, d_in_stride, nbits, m_nchans, st.d_rows.as<uint32_t>(),
+    DD_HIP(transpose_rows(st.fast && dd_tdd_tiling_is_planes(st.tiling), d_in, nsamps, d_in_stride, nbits, m_nchans, st.d_rows.as<uint32_t>(),
                             st.row_words, stream));
     ctx.timer.end(StageTimer::UNPACK, stream);
 
@@ -597,8 +767,8 @@ void TDDPlan::execute_span(size_type nsamps, const byte_type* in, size_type in_n
             // the tables of DM block b0 / (waves * dms_per_wave) start at DM b0
             const size_t b0blk = b0 / ((size_t)st.tiling.waves * st.tiling.dms_per_wave);
             DD_HIP(dd_tdd_dedisperse_lds(st.d_rows.as<uint32_t>(), st.row_words, nbits,
-                                         st.d_code.as<uint32_t>() + b0 * st.nact, st.d_chan.as<int32_t>(),
-                                         st.d_wstart.as<uint32_t>() + b0blk * st.nact,
+                                         st.d_code.as<uint32_t>() + b0 * st.code_per_dm, st.d_chan.as<int32_t>(),
+                                         st.d_wstart.as<uint32_t>() + b0blk * st.wstart_per_blk,
                                          st.d_chunks.as<uint32_t>() + b0blk * st.maxc, st.maxc, st.nact, nb,
                                          nsc, d_out + b0 * d_out_stride, d_out_stride, ep, st.tiling, stream));
         } else {
@@ -673,24 +843,37 @@ void TDDPlan::execute_noalloc(size_type nsamps, const byte_type* in, size_type i
     ctx.make_current();
     hipStream_t stream = ctx.exec;
     const unsigned nbits = (unsigned)in_nbits;
-    prepare_tables(nbits, 0, m_dm_count, /*upload=*/false);
-    const size_t row_words = row_words_for(nbits, nsamps, nsc);
-
     // scratch layout: delay codes (64 spare entries), channels, weights,
     // window starts, then the transposed rows; 256-byte aligned pieces
-    size_t used = 0;
-    auto carve = [&](size_t bytes) {
-        const size_t at = used;
-        used += round_up(std::max<size_t>(bytes, 4), 256);
-        return at;
+    size_t used = 0, row_words = 0;
+    size_t o_code = 0, o_chan = 0, o_weight = 0, o_wstart = 0, o_chunks = 0, o_rows = 0;
+    auto lay_out = [&](bool packed) {
+        prepare_tables(nbits, 0, m_dm_count, /*upload=*/false, packed);
+        row_words = row_words_for(nbits, nsamps, nsc);
+        used = 0;
+        auto carve = [&](size_t bytes) {
+            const size_t at = used;
+            used += round_up(std::max<size_t>(bytes, 4), 256);
+            return at;
+        };
+        o_code = carve((st.h_tab.size() + 64) * 4);
+        o_chan = carve((st.nact + 8) * 4);
+        o_weight = carve(st.nact * 4);
+        o_wstart = carve((st.h_wstart.size() + 8) * 4);
+        o_chunks = carve(st.h_chunks.size() * 4);
+        o_rows = carve(m_nchans * row_words * 4);
+        return used <= scratch_bytes;
     };
-    const size_t o_code = carve((st.h_tab.size() + 64) * 4);
-    const size_t o_chan = carve((st.nact + 8) * 4);
-    const size_t o_weight = carve(st.nact * 4);
-    const size_t o_wstart = carve((st.h_wstart.size() + 8) * 4);
-    const size_t o_chunks = carve(st.h_chunks.size() * 4);
-    const size_t o_rows = carve(m_nchans * row_words * 4);
-    if (used > scratch_bytes) DD_THROW(DEDISP_MEM_ALLOC_FAILED);
+    // bit-plane rows take whole tiles: where they do not fit, the packed-lane
+    // layout (and its tables) may, and is kept for the series length
+    const std::array<uint64_t, 3> packed_key = {m_tables_version, nbits, nsamps};
+    const bool few = !st.tuned[nbits].waves && too_few_for_planes(nbits, planes_tiles(nsc), m_dm_count);
+    if (few || st.noalloc_packed == packed_key) {
+        if (!lay_out(true)) DD_THROW(DEDISP_MEM_ALLOC_FAILED);
+    } else if (!lay_out(false)) {
+        if (!dd_tdd_tiling_is_planes(st.tiling) || !lay_out(true)) DD_THROW(DEDISP_MEM_ALLOC_FAILED);
+        st.noalloc_packed = packed_key;
+    }
     uint8_t* const base = static_cast<uint8_t*>(scratch);
     auto* d_code = reinterpret_cast<uint32_t*>(base + o_code);
     auto* d_chan = reinterpret_cast<int32_t*>(base + o_chan);
@@ -722,7 +905,7 @@ void TDDPlan::execute_noalloc(size_type nsamps, const byte_type* in, size_type i
     // the transpose writes every word of every row (zero beyond the data), so
     // nothing in the scratch needs clearing
     const size_t row_bytes = (m_nchans * nbits + 7) / 8;
-    DD_HIP(dd_tdd_transpose(in, nsamps, row_bytes, nbits, m_nchans, d_rows, row_words, stream));
+    DD_HIP(transpose_rows(st.fast && dd_tdd_tiling_is_planes(st.tiling), in, nsamps, row_bytes, nbits, m_nchans, d_rows, row_words, stream));
     const size_t out_stride = nsc * (out_nbits / 8);
     const dd_tdd_epilogue ep = make_epilogue(nbits, out_nbits, m_nchans);
     if (st.fast)
@@ -761,7 +944,10 @@ void TDDPlan::execute_batch(size_type nbeams, const size_type* nsamps, const byt
     TDDState& st = *m_state;
     ctx.make_current();
     hipStream_t stream = ctx.exec;
-    prepare_tables(nbits, 0, m_dm_count);
+    size_t tiles = 0;
+    for (size_t b = 0; b < nbeams; ++b) tiles += planes_tiles(nsamps[b] - m_max_delay);
+    prepare_tables(nbits, 0, m_dm_count, true,
+                   !st.tuned[nbits].waves && too_few_for_planes(nbits, tiles, m_dm_count));
     if (!st.fast || st.nact == 0) {
         // weighted killmask or 16/32-bit samples: one beam after another
         for (size_t b = 0; b < nbeams; ++b)
@@ -865,7 +1051,7 @@ void TDDPlan::execute_batch(size_type nbeams, const size_type* nsamps, const byt
         if (timed) ctx.timer.begin(StageTimer::UNPACK, stream);
         for (size_t b = 0; b < nbeams; ++b) {
             const uint8_t* src = device_ptrs ? in[b] : bin + ioff[b];
-            DD_HIP(dd_tdd_transpose(src, nsamps[b], row_bytes, nbits, m_nchans,
+            DD_HIP(transpose_rows(st.fast && dd_tdd_tiling_is_planes(st.tiling), src, nsamps[b], row_bytes, nbits, m_nchans,
                                     st.d_brows.as<uint32_t>() + roff[b], rw[b], stream));
         }
         if (timed) ctx.timer.end(StageTimer::UNPACK, stream);

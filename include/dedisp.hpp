@@ -185,7 +185,7 @@ private:
                       byte_type* out, size_type out_nbits, size_type out_stride, dedisp_size first_dm_idx,
                       dedisp_size dm_count, unsigned flags);
     void prepare_tables(unsigned nbits, dedisp_size first_dm_idx, dedisp_size dm_count,
-                        bool upload = true);
+                        bool upload = true, bool packed = false);
     size_t row_words_for(unsigned nbits, size_t nsamps, size_t nsc) const;
 
     dedisp_size m_gulp_size;

@@ -269,3 +269,23 @@ def test_fdd_cpu_asis_matches_its_fp64_formula(orc):
     # transform are filled, which low-passes the output even at DM 0.
     ts = orc.fdd_timeseries(nch, delays, dms, nsamps, maxd, data)
     assert np.linalg.norm(got[0] - ts[0]) / np.linalg.norm(ts[0]) > 0.1
+
+
+@pytest.mark.parametrize("vmax", [1, 3, 15, 255])
+@pytest.mark.parametrize("out_range", [1, 255, 65535])
+def test_quotient_from_the_reciprocal(vmax, out_range):
+    """The bit-plane kernel's epilogue divides by multiplying with the rounded
+    reciprocal and correcting once with the exact remainder: the IEEE quotient
+    for every sum. Channel counts around powers of two and at random; the
+    remainder is exact in 64 bits, the corrected sum in extended precision."""
+    rng = np.random.default_rng(vmax + out_range)
+    for nch in {1, 2, 3, 5, 7, 63, 64, 65, 460, 511, 512, 513, 1023, 1024, 8191, 8192, *rng.integers(1, 8193, 12)}:
+        den = np.float32(vmax * int(nch))
+        top = vmax * int(nch)
+        s = np.arange(top + 1) if top < 60000 else np.unique(rng.integers(0, top + 1, 60000))
+        num = s.astype(np.float32) * np.float32(out_range)
+        rcp = np.float32(1) / den
+        q = num * rcp
+        r = (num.astype(np.float64) - q.astype(np.float64) * np.float64(den)).astype(np.float32)
+        got = (q.astype(np.longdouble) + r.astype(np.longdouble) * np.longdouble(rcp)).astype(np.float32)
+        assert np.array_equal(got, num / den), nch

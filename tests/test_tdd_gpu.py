@@ -437,3 +437,136 @@ def test_tdd_gulped_execution_matches_resident(dd, orc, gulp, nbits, out_nbits):
     r = orc.tdd(nch, delays, None, dms, nsamps, plan.max_delay, data, nbits, out_nbits, first_dm=96, dm_count=1)
     assert np.array_equal(got[96], r[0])
     assert dd.lib().dedisp_set_gulp_size(plan.handle, 0) == dd.DEDISP_UNKNOWN_ERROR
+
+
+PLANES_SHAPES = [(1, "2,8"), (1, "1,8"), (2, "2,8"), (2, "1,8"), (4, "2,8"), (4, "1,8"), (8, "1,8")]
+
+
+@pytest.mark.parametrize("nbits,shape", PLANES_SHAPES)
+@pytest.mark.parametrize("nch,nout,ndm,dm_hi,out_nbits", [
+    (64, 1, 1, 0.0, 32),          # one output, one DM
+    (72, 4096, 17, 3.0, 32),      # a whole tile of outputs, a block and one DM
+    (200, 4097, 33, 61.0, 8),     # one output past a tile
+    (40, 8191, 40, 60.0, 16),     # partly filled chunk, delays within a tile
+    (136, 12345, 24, 900.0, 32),  # windows that start several tiles on, killed channels
+])
+def test_tdd_planes_kernel_vs_oracle(dd, orc, monkeypatch, nbits, shape, nch, nout, ndm, dm_hi, out_nbits):
+    """The bit-plane kernel over the edges of its tiles (4096 outputs), chunks
+    and DM blocks; whole sums, so the outputs are the oracle's."""
+    monkeypatch.setenv("DEDISP_TDD_TILING", f"64,{shape},16")
+    geom = (64e-6, 1500.0, -400.0 / nch)
+    dms = np.linspace(0, dm_hi, ndm, dtype=f32)
+    delays = orc.delay_table(nch, f32(geom[0]), f32(geom[1]), f32(geom[2]))
+    md = orc.max_delay(float(dms[-1]), float(delays[-1]))
+    km = np.ones(nch, np.int32)
+    if ndm == 24:
+        km[::5] = 0
+    out, ref = _random_case(dd, orc, nbits, nch, nout + md, dms, seed=nbits + nout, geom=geom, killmask=km,
+                            out_nbits=out_nbits)
+    assert out.shape[1] == nout
+    assert np.array_equal(out, ref)
+
+
+@pytest.mark.parametrize("nbits,nact", [(1, 1023), (1, 1024), (2, 682), (2, 683), (4, 1092), (4, 1093), (8, 64),
+                                        (8, 65), (8, 257), (8, 258), (8, 1028), (8, 1029)])
+def test_tdd_planes_kernel_largest_sums(dd, orc, monkeypatch, nbits, nact):
+    """All samples at their largest value, with the channel counts at which the
+    counters take another plane."""
+    monkeypatch.setenv("DEDISP_TDD_TILING", "64,1,8,16" if nbits == 8 else "64,2,8,16")
+    dt, f0, df = 64e-6, 1500.0, -0.1
+    nch = (nact + 7) // 8 * 8
+    km = (np.arange(nch) < nact).astype(np.int32)
+    plan = dd.Plan(nch, dt, f0, df, impl=dd.TDD)
+    plan.set_killmask(km)
+    dms = np.linspace(0, 20, 9, dtype=f32)
+    plan.set_dm_list(dms)
+    nsamps = 4500 + plan.max_delay
+    s = np.full((nsamps, nch), (1 << nbits) - 1, np.uint8)
+    s[::97, ::3] = 0
+    data = dd.pack_samples(s, nbits)
+    out = plan.execute(data, nbits, 32)
+    delays = orc.delay_table(nch, f32(dt), f32(f0), f32(df))
+    assert np.array_equal(out, orc.tdd(nch, delays, km, dms, nsamps, plan.max_delay, data, nbits, 32))
+    plan.close()
+
+
+@pytest.mark.parametrize("nbits", [1, 2, 4, 8])
+@pytest.mark.parametrize("step", [75, 160, 330])
+def test_tdd_planes_wide_windows(dd, orc, nbits, step):
+    """Delays that lie up to step samples apart from DM to DM: 2 DMs per wave, 1
+    DM per wave with more LDS, and windows for the packed-lane kernels."""
+    nch, geom = 40, (64e-6, 1500.0, -10.0)
+    delays = orc.delay_table(nch, f32(geom[0]), f32(geom[1]), f32(geom[2]))
+    dms = (np.arange(100) * (step / float(delays[-1]))).astype(f32)
+    md = orc.max_delay(float(dms[-1]), float(delays[-1]))
+    out, ref = _random_case(dd, orc, nbits, nch, 50001 + md, dms, seed=step + nbits, geom=geom)
+    assert np.array_equal(out, ref)
+
+
+@pytest.mark.parametrize("nbits,nch,ndm", [(1, 40, 400), (2, 40, 400), (4, 34, 400), (8, 33, 700)])
+def test_tdd_kernel_follows_the_size(dd, orc, nbits, nch, ndm):
+    """One plan for a long series, a short one, the long one again and a range
+    of its DMs: launches on both sides of the bit-plane kernel's rule, each with
+    its own tables."""
+    geom = (64e-6, 1500.0, -400.0 / nch)
+    plan = _plan(dd, nch, *geom)
+    dms = np.linspace(0, 120, ndm, dtype=f32)
+    plan.set_dm_list(dms)
+    delays = orc.delay_table(nch, f32(geom[0]), f32(geom[1]), f32(geom[2]))
+    rng = np.random.default_rng(nbits)
+    md = plan.max_delay
+    for nsamps in (md + 24000, md + 1500, md + 24000):
+        s = rng.integers(0, 1 << nbits, size=(nsamps, nch)).astype(np.uint8)
+        data = dd.pack_samples(s, nbits)
+        out = plan.execute(data, nbits, 32)
+        assert np.array_equal(out, orc.tdd(nch, delays, None, dms, nsamps, md, data, nbits, 32)), nsamps
+    part = plan.execute(dd.pack_samples(s, nbits), nbits, 16)
+    assert np.array_equal(part, orc.tdd(nch, delays, None, dms, nsamps, md, data, nbits, 16))
+    plan.close()
+
+
+def test_tdd_planes_batch_replays(dd):
+    """A batch large enough for the bit-plane kernel (a captured graph) against
+    single executes, new contents in the same buffers on every replay."""
+    import torch
+    nch, nbits = 40, 2
+    plan = dd.Plan(nch, 64e-6, 1500.0, -10.0, impl=dd.TDD)
+    plan.set_dm_list(np.linspace(0, 100, 300, dtype=f32))
+    md, ndm = plan.max_delay, plan.dm_count
+    lengths = [md + 20001, md + 1, md + 4096, md + 9000]
+    rng = np.random.default_rng(9)
+    d_in = [torch.zeros((n, nch * nbits // 8), dtype=torch.uint8, device="cuda") for n in lengths]
+    d_out = [torch.empty((ndm, n - md), dtype=torch.float32, device="cuda") for n in lengths]
+    for rep in range(4):
+        host = [dd.pack_samples(rng.integers(0, 4, size=(n, nch)).astype(np.uint8), nbits) for n in lengths]
+        for t, h in zip(d_in, host):
+            t.copy_(torch.from_numpy(h))
+        torch.cuda.synchronize()
+        assert plan.execute_batch_raw(lengths, d_in, nbits, d_out, 32, dd.DEVICE_POINTERS) == 0
+        torch.cuda.synchronize()
+        for o, h, n in zip(d_out, host, lengths):
+            if n > md:
+                assert np.array_equal(o.cpu().numpy(), plan.execute(h, nbits, 32)), (rep, n)
+    plan.close()
+
+
+def test_tdd_planes_noalloc_at_the_scratch_limit(dd):
+    """Bit-plane rows take whole tiles: a series whose packed rows just fit the
+    fixed scratch is still accepted, one that fits either way runs on planes."""
+    import torch
+    nch, nbits = 1024, 4
+    plan = dd.Plan(nch, 64e-6, 1530.0, -0.3125, impl=dd.TDD)
+    plan.set_dm_list(np.linspace(0, 20, 64, dtype=f32))
+    # 4096-sample tiles of 512-byte samples: 63 + 2 of them exceed 128 MiB
+    n_limit = 255_000
+    assert n_limit * nch // 2 < dd.NOALLOC_SCRATCH_BYTES < 65 * 4096 * nch // 2
+    for n in (n_limit, 200_000, n_limit):
+        d_in = torch.randint(0, 256, (n, nch // 2), dtype=torch.uint8, device="cuda")
+        a = torch.empty((plan.dm_count, n - plan.max_delay), dtype=torch.float32, device="cuda")
+        b = torch.empty_like(a)
+        torch.cuda.synchronize()
+        assert plan.execute_noalloc_raw(n, d_in, nbits, a, 32, 0) == 0
+        assert plan.execute_raw(n, d_in, nbits, b, 32, dd.DEVICE_POINTERS) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(a, b), n
+    plan.close()
