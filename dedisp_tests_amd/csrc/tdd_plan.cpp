@@ -655,8 +655,9 @@ void TDDPlan::execute_guru(size_type nsamps, const byte_type* in, size_type in_n
         if (m_max_delay + 65536 > kMaxSpan) DD_THROW(DEDISP_UNKNOWN_ERROR);
         gulp = kMaxSpan - m_max_delay;
     }
-    {
-        m_ctx->make_current();
+    // (never less than 65536: a shorter one needs no look at the free memory)
+    m_ctx->make_current();
+    if (gulp > 65536) {
         size_t free_b = 0, total_b = 0;
         DD_HIP(hipMemGetInfo(&free_b, &total_b));
         auto need = [&](size_t g) {
