@@ -156,7 +156,11 @@ constexpr uint32_t low_blocks_mask(int sh)
     return m;
 }
 
-template <int NBITS>
+//
+// TS sample rows per tile: 256, or 64 where the launch would have fewer than
+// two workgroups per CU (64 ch x 8192 8-bit samples: 37 workgroups, 12.8 us, one
+// loading its 64-byte rows word after word; 148 and all loads in flight 3.2 us).
+template <int NBITS, int TS>
 __global__ __launch_bounds__(256) void tdd_transpose_reg_k(
     const uint8_t* __restrict__ in, size_t nsamps, size_t in_stride, size_t row_bytes,
     size_t nchans, uint32_t* __restrict__ out, size_t row_words)
@@ -164,29 +168,34 @@ __global__ __launch_bounds__(256) void tdd_transpose_reg_k(
     static_assert(NBITS == 2 || NBITS == 4 || NBITS == 8, "register transpose: 2-, 4- or 8-bit");
     constexpr int SPW = 32 / NBITS;          // samples per output word = channels per row word
     constexpr int RW = TR_CB / 4;            // words per tile row (32)
-    constexpr int WPC = TR_TS / SPW;         // output words per channel per tile
-    __shared__ __attribute__((aligned(16))) uint32_t tile[TR_TS * RW];
+    constexpr int WPC = TS / SPW;            // output words per channel per tile
+    __shared__ __attribute__((aligned(16))) uint32_t tile[TS * RW];
 
-    const size_t t0 = (size_t)blockIdx.x * TR_TS;
+    const size_t t0 = (size_t)blockIdx.x * TS;
     const size_t b0 = (size_t)blockIdx.y * TR_CB;
     const int tid = threadIdx.x;
     auto slot = [](int t, int d) { return t * RW + (d ^ ((t / SPW) & (RW - 1))); };
 
     const bool words = ((in_stride | reinterpret_cast<uintptr_t>(in)) & 3u) == 0;
-    if (words && t0 + TR_TS <= nsamps && b0 + TR_CB <= row_bytes) {
-        // interior tile: every load in bounds, all issued before the first is
-        // waited on (thread tid takes word tid % 32 of rows tid / 32 + 8k)
-        constexpr int PER = TR_TS * RW / 256;
+    if (words && t0 + TS <= nsamps && row_bytes % 4 == 0) {
+        // whole words of whole rows: a thread's word lies in the row or beyond
+        // it (zeros); all its loads are issued before the first is waited on
+        // (thread tid takes word tid % 32 of rows tid / 32 + 8k)
+        constexpr int PER = TS * RW / 256;
         const int d = tid % RW, tl0 = tid / RW;
         const uint8_t* src = in + (t0 + tl0) * in_stride + b0 + 4 * d;
         uint32_t v[PER];
 #pragma unroll
-        for (int k = 0; k < PER; ++k)
-            v[k] = *reinterpret_cast<const uint32_t*>(src + (size_t)(8 * k) * in_stride);
+        for (int k = 0; k < PER; ++k) v[k] = 0;
+        if (b0 + 4 * d < row_bytes) {
+#pragma unroll
+            for (int k = 0; k < PER; ++k)
+                v[k] = *reinterpret_cast<const uint32_t*>(src + (size_t)(8 * k) * in_stride);
+        }
 #pragma unroll
         for (int k = 0; k < PER; ++k) tile[slot(tl0 + 8 * k, d)] = v[k];
     } else {
-        for (int i = tid; i < TR_TS * RW; i += 256) {
+        for (int i = tid; i < TS * RW; i += 256) {
             const int tl = i / RW, d = i % RW;
             const size_t t = t0 + tl, b = b0 + 4 * (size_t)d;
             uint32_t v = 0;
@@ -599,18 +608,26 @@ extern "C" hipError_t dd_tdd_transpose(const uint8_t* in, size_t nsamps, size_t 
     const size_t row_bytes = (nchans * nbits + 7) / 8;
     const size_t spw = 32 / nbits;
     const size_t total_samps = row_words * spw;
-    dim3 grid((unsigned)((total_samps + TR_TS - 1) / TR_TS),
-              (unsigned)((row_bytes + TR_CB - 1) / TR_CB));
+    const unsigned gy = (unsigned)((row_bytes + TR_CB - 1) / TR_CB);
+    const dim3 grid((unsigned)((total_samps + TR_TS - 1) / TR_TS), gy);
+    const dim3 grid64((unsigned)((total_samps + 63) / 64), gy);
+    const bool small = (size_t)grid.x * gy < 512;
     const size_t rb = (in_stride < row_bytes) ? in_stride : row_bytes;
+#define DD_TRANSPOSE(NB)                                                                                              \
+    if (small) hipLaunchKernelGGL((tdd_transpose_reg_k<NB, 64>), grid64, dim3(256), 0, stream, in, nsamps, in_stride, \
+                                  rb, nchans, out, row_words);                                                        \
+    else hipLaunchKernelGGL((tdd_transpose_reg_k<NB, TR_TS>), grid, dim3(256), 0, stream, in, nsamps, in_stride, rb,  \
+                            nchans, out, row_words)
     switch (nbits) {
     case 1:  hipLaunchKernelGGL(tdd_transpose_k<1>, grid, dim3(256), 0, stream, in, nsamps, in_stride, rb, nchans, out, row_words); break;
-    case 2:  hipLaunchKernelGGL(tdd_transpose_reg_k<2>, grid, dim3(256), 0, stream, in, nsamps, in_stride, rb, nchans, out, row_words); break;
-    case 4:  hipLaunchKernelGGL(tdd_transpose_reg_k<4>, grid, dim3(256), 0, stream, in, nsamps, in_stride, rb, nchans, out, row_words); break;
-    case 8:  hipLaunchKernelGGL(tdd_transpose_reg_k<8>, grid, dim3(256), 0, stream, in, nsamps, in_stride, rb, nchans, out, row_words); break;
+    case 2:  DD_TRANSPOSE(2); break;
+    case 4:  DD_TRANSPOSE(4); break;
+    case 8:  DD_TRANSPOSE(8); break;
     case 16: hipLaunchKernelGGL(tdd_transpose_k<16>, grid, dim3(256), 0, stream, in, nsamps, in_stride, rb, nchans, out, row_words); break;
     case 32: hipLaunchKernelGGL(tdd_transpose_k<32>, grid, dim3(256), 0, stream, in, nsamps, in_stride, rb, nchans, out, row_words); break;
     default: return hipErrorInvalidValue;
     }
+#undef DD_TRANSPOSE
     return hipGetLastError();
 }
 

@@ -103,15 +103,16 @@ __global__ __launch_bounds__(256) void tdd_transpose_planes_k(
     const bool words = ((in_stride | reinterpret_cast<uintptr_t>(in)) & 3u) == 0;
     const int w = tid % TP_W, row0 = tid / TP_W;
     const size_t b = b0 + 4 * (size_t)w;
-    if (words && b0 + TP_W * 4 <= row_bytes && tq + 31 * T + TP_P <= nsamps) {
-        // every load in bounds: 16 issued before the first is waited on
+    if (words && row_bytes % 4 == 0 && tq + 31 * T + TP_P <= nsamps) {
+        // whole words of whole rows: a thread's word lies in the row or beyond
+        // it (zeros); 16 loads are issued before the first is waited on
         for (int n0 = 0; n0 < 64; n0 += 16) {
             uint32_t v[16];
 #pragma unroll
             for (int n = 0; n < 16; ++n) {
                 const int row = row0 + 16 * (n0 + n);  // run row / 32, position row % 32
                 const size_t t = tq + (size_t)(row / TP_P) * T + row % TP_P;
-                v[n] = *reinterpret_cast<const uint32_t*>(in + t * in_stride + b);
+                v[n] = (b < row_bytes) ? *reinterpret_cast<const uint32_t*>(in + t * in_stride + b) : 0;
             }
 #pragma unroll
             for (int n = 0; n < 16; ++n) tile[(row0 + 16 * (n0 + n)) * (TP_W + 1) + w] = v[n];
