@@ -680,26 +680,9 @@ __global__ __launch_bounds__(WAVES * 64, 512 / (WAVES * 64)) void fdd_mfma16_k(
         load_half(0, 1);
         store_half(xs, 1);
         APl A0, A1;
-        const bool idle = dmw >= ndm;  // wave-uniform: no DM of this wave exists
-        if (!idle) {
 #pragma unroll
-            for (int pc = 0; pc < MT * 4; ++pc) gen_piece(k0, A0, pc);
-        }
+        for (int pc = 0; pc < MT * 4; ++pc) gen_piece(k0, A0, pc);
         __syncthreads();
-        // A wave past the last DM only stages, leaving its SIMD's issue slots
-        // and matrix cores to the others (777 DMs are 3 whole blocks and 9 rows)
-        if (idle) {
-            for (uint32_t ks = 0; ks < nks; ++ks) {
-                const size_t kn = (ks + 1 < nks) ? ks + 1 : ks;
-                char* nbuf = xs + ((ks + 1) & 1) * BUF;
-                load_half(kn * kstep_p, 0);
-                store_half(nbuf, 0);
-                load_half(kn * kstep_p, 1);
-                store_half(nbuf, 1);
-                __syncthreads();
-            }
-            return;
-        }
         for (uint32_t ks = 0; ks < nks; ++ks) {
             const uint32_t kn = (ks + 1 < nks) ? ks + 1 : ks;
             load_half((size_t)kn * kstep_p, 0);

@@ -380,7 +380,7 @@ size_t FDDGPUPlan::segment_length(const size_t* nsc, size_t n) const
         // Contraction: a chunk group of ntl 8-chunk tiles costs ntl tiles of
         // products plus the phasors, kPhasorTiles tiles' worth whatever its
         // width (1024 ch x 2048 DMs x 65536: one tile 20.9 ms, three 38.5 ms),
-        // for every bin, channel and DM, the DMs in whole waves of 32.
+        // for every bin, channel and DM.
         // Transforms: one per chunk and channel, one per chunk and DM.
         // The smallest volume of columns x bins, which this replaces, left out
         // phasors and transforms and took 131072 and one tile of 5 chunks at
