@@ -24,15 +24,16 @@
 // The counters hold the exact sums (the uint32 sums of
 // src/tdd/dedisperse/dedisperse_kernel.cuh:151-193).
 //
-// What bounds it is the bit operations (half-rate) and, where the delays of a
-// block's DMs spread over several times T, the staging. Execute times, packed
+// What bounds it is the bit operations (half-rate) and the staging: every block
+// of DMs fetches its windows of every channel, 26.6 GB a launch at the 4-bit
+// size below (1.9 TB/s). Execute times, packed
 // lanes (4-bit: runs layout) -> planes: 1-bit 512 ch x 200003 x 501 DMs 0.99 ->
 // 0.35 ms; 2-bit 512 ch x 4 beams (2.4e6 samples) x 1024 DMs 21.8 -> 8.4 ms;
-// 4-bit 1024 ch x 2^20 x 1167 DMs 22.9 -> 15.8 ms (14.8 on another box); 8-bit
-// 1024 ch x 15625 x 3000 DMs 1.92 -> 1.45 ms. Tried: 4 DMs per wave (spills),
+// 4-bit 1024 ch x 2^20 x 1167 DMs 22.9 -> 14.6 ms; 8-bit 1024 ch x 15625 x 3000
+// DMs 1.92 -> 1.43 ms. Tried: 4 DMs per wave (spills),
 // staging each position with two loads of its own (2-bit 11.6 ms), its scalar
-// loads where they are used (10.0 ms), the carries of four chunks together
-// (4-bit spills: 19.7 ms).
+// loads where they are used (10.0 ms), the carries of four chunks together (14 %
+// fewer bit operations, 4-bit unchanged).
 #include <hip/hip_runtime.h>
 
 #include "kernels.h"
@@ -367,13 +368,22 @@ __global__ __launch_bounds__(WAVES * 64, 4) void tdd_planes_k(
         for (int n = 0; n < IPW; ++n) d[n] = desc[ci * CC + item_of(n) / G];
         P = pos[ci];
     };
-    auto stage_load = [&](const uint2 (&d)[IPW]) {
+    // The third word is needed (and lies in another tile's cache lines) only
+    // where the window's runs pass the next tile's start. 4- and 8-bit input
+    // loads the second again elsewhere (4-bit, 1024 ch x 2^20 x 1167 DMs: 21.4
+    // instead of 39 GB fetched, 15.07 -> 14.55 ms); with the fewer bytes and
+    // more items of 1- and 2-bit input finding out costs more (2-bit 8.30 ->
+    // 8.63 ms).
+    auto stage_load = [&](const uint2 (&d)[IPW], uint32_t P) {
 #pragma unroll
         for (int n = 0; n < IPW; ++n) {
             gword* src = (gword*)rows + (size_t)d[n].y * row_words + ((size_t)tile + d[n].x / T / 32) * (T * NB) +
                          (64 * (item_of(n) % G) + lane) * NB;
-#pragma unroll
-            for (int k = 0; k < 3; ++k) load_planes<NB>(src + k * (T * NB), w[n][k]);
+            const uint32_t a = d[n].x;
+            const uint32_t third = (NB < 4 || a / T % 32 + (a % T + P + T - 1) / T > 32) ? 2 : 1;
+            load_planes<NB>(src, w[n][0]);
+            load_planes<NB>(src + T * NB, w[n][1]);
+            load_planes<NB>(src + third * (T * NB), w[n][2]);
         }
     };
     auto stage_write = [&](const uint2 (&d)[IPW], uint32_t P) {
@@ -414,7 +424,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void tdd_planes_k(
     uint2 dc[IPW], dn[IPW];  // descriptors of this chunk's and the next one's items
     uint32_t Pc, Pn;
     load_desc(0, dc, Pc);
-    stage_load(dc);
+    stage_load(dc, Pc);
     // Chunk ci, ci % 2 = PH (the number of chunks is even). The carry of an even
     // chunk into plane LT waits for the odd one's (one full adder for both), so
     // that the half adders through the planes above run once in two chunks.
@@ -446,7 +456,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void tdd_planes_k(
         asm volatile("" : "+s"(Pn));
         Pc = Pn;
         __syncthreads();
-        stage_load(dc);  // (the last chunk's again after the last one)
+        stage_load(dc, Pc);  // (the last chunk's again after the last one)
         // all LDS words of a step first, so that their latencies overlap
         constexpr int KB = (NB < 4 && 2 * CC * NB <= 32) ? 2 : 1;
 #pragma unroll
