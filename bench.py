@@ -160,7 +160,8 @@ def cpu_baseline(seconds_budget: float = 30.0):
     }
 
 
-MFMA_PEAK_T = {"fp32": 157.3, "bf16": 2500.0, "fp16": 2500.0}   # dense TFLOP/s
+# dense TFLOP/s; the float32 form runs on float16 products (hi + lo pairs, three each)
+MFMA_PEAK_T = {"fp32": 2500.0, "bf16": 2500.0, "fp16": 2500.0}
 
 
 def mfma16_tiles(nchunk: int) -> tuple:
@@ -277,7 +278,7 @@ def fdd_leg(torch, dd, steps: int, warmup: int, forms=("fp32", "bf16", "fp16"), 
                                  "bins 0..nfft/2 (no padding, no compensation products); the kernel time is "
                                  "measured with HIP events on the plan's stream over the timed executes"},
         }
-        if name == "bf16":
+        if name in ("bf16", "fp32"):
             # matrix-core work the kernel issues: three products per complex
             # multiply-add (hi x hi, hi x lo, lo x hi) over chunk groups padded
             # to 8-chunk N-tiles
@@ -779,7 +780,7 @@ def tdd_leg(torch, dd, steps: int, warmup: int) -> tuple:
         "roofline": {"bound": "hbm", "achieved": achieved_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved_gbs / HBM_PEAK_GBS, "traffic": measured_traffic(),
                      "traffic_source": "profiles/tdd-1024ch-2p20x4bit-1167dm_hbm-traffic.md",
-                     "kernel": "tdd_runs_k", "kernel_ms": k_ms, "algorithmic_bytes": in_bytes + out_bytes,
+                     "kernel": "tdd_planes_k", "kernel_ms": k_ms, "algorithmic_bytes": in_bytes + out_bytes,
                      "note": "LDS reads and VALU issue bound this kernel, not HBM: see valu_roofline"},
         "valu_roofline": valu_roofline(k_ms, adds_t),
         "stages_ms": {"transpose": float(np.mean(unpack_ms)), "channel_sum": k_ms},
@@ -883,7 +884,7 @@ def main():
     peaks = peaks_leg(torch)
     line["measured_peaks"] = peaks
     line["roofline"]["frac_of_measured_gemm"] = line["roofline"]["achieved"] / peaks["bf16_gemm_tflops"]
-    for form, key in (("fp32", "fp32_gemm_tflops"), ("fp16", "fp16_gemm_tflops")):
+    for form, key in (("fp32", "fp16_gemm_tflops"), ("fp16", "fp16_gemm_tflops")):
         if form in line["fdd"]:
             rl = line["fdd"][form]["roofline"]
             rl["frac_of_measured_gemm"] = rl["achieved"] / peaks[key]
