@@ -37,6 +37,7 @@
 #include <hip/hip_runtime.h>
 
 #include "kernels.h"
+#include "tdd_planes_stage.h"
 
 namespace {
 
@@ -379,8 +380,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void tdd_planes_k(
         for (int n = 0; n < IPW; ++n) {
             gword* src = (gword*)rows + (size_t)d[n].y * row_words + ((size_t)tile + d[n].x / T / 32) * (T * NB) +
                          (64 * (item_of(n) % G) + lane) * NB;
-            const uint32_t a = d[n].x;
-            const uint32_t third = (NB < 4 || a / T % 32 + (a % T + P + T - 1) / T > 32) ? 2 : 1;
+            const uint32_t third = (NB < 4 || planes_needs_third(d[n].x, P)) ? 2 : 1;
             load_planes<NB>(src, w[n][0]);
             load_planes<NB>(src + T * NB, w[n][1]);
             load_planes<NB>(src + third * (T * NB), w[n][2]);
@@ -390,29 +390,13 @@ __global__ __launch_bounds__(WAVES * 64, 4) void tdd_planes_k(
 #pragma unroll
         for (int n = 0; n < IPW; ++n) {
             const uint32_t item = item_of(n);
-            const uint32_t a = d[n].x;
-            const uint32_t r0 = a / T % 32;
-            const uint32_t nu = max((a % T + P + T - 1) / T, 1u);
-            // position in the window of this lane's first word (negative, as a
-            // large unsigned, before its start)
-            const uint32_t s = 64 * (item % G) + lane - a % T;
-            uint32_t* const dst = lds + ((item / G) * stride + s) * NB;
-            auto put = [&](int k, uint32_t u, bool in) {
+            const uint32_t a = d[n].x, p = 64 * (item % G) + lane;
+            planes_stage(a, P, p, [&](int k, uint32_t shift, uint32_t u, bool in) {
                 uint32_t v[NB];
 #pragma unroll
-                for (int b = 0; b < NB; ++b) v[b] = __builtin_amdgcn_alignbit(w[n][k + 1][b], w[n][k][b], r0 + u);
-                if (in) write_planes<NB>(dst + u * (T * NB), v);
-            };
-            // only the first and the last word of a lane may lie outside; from
-            // u = 32 - r0 on the runs start in the next tile
-            const uint32_t last = nu - 1, u1 = min(last, 32 - r0);
-            put(0, 0, s < P);
-            for (uint32_t u = 1; u < u1; ++u) put(0, u, true);
-            for (uint32_t u = max(u1, 1u); u < last; ++u) put(1, u, true);
-            if (nu > 1) {
-                if (r0 + last < 32) put(0, last, s + last * T < P);
-                else put(1, last, s + last * T < P);
-            }
+                for (int b = 0; b < NB; ++b) v[b] = __builtin_amdgcn_alignbit(w[n][k + 1][b], w[n][k][b], shift);
+                if (in) write_planes<NB>(lds + planes_lds_word(item / G, stride, planes_window_pos(a, p, u), NB), v);
+            });
         }
     };
 
