@@ -161,6 +161,17 @@ hipError_t dd_fdd_contract_mfma16(int prec, int mirror, const float2* X, size_t 
 // nchunk chunks, and the number of chunk groups.
 int dd_fdd_mfma16_tiles(size_t nchunk, int prec, int* ntl, size_t* ngroups);
 
+// DMs a workgroup of the matrix-core contractions computes, whole or in part.
+#define DD_FDD_DM_BLOCK 256
+
+// Automatic overlap-save segment length (host only) for series with
+// nsc[0..n) outputs per DM, largest delay dmax, ndm DMs and nchan channels: a
+// supported length (2^13 .. 2^18) above dmax + 3, 0 when there is none. form 0
+// = vector-ALU contraction, 1 = 32 x 32 tiles, 2 = 16 x 16 tiles; prec as in
+// dd_fdd_contract_mfma16.
+size_t dd_fdd_segment_length(int form, int prec, size_t dmax, const size_t* nsc, size_t n, size_t ndm,
+                             size_t nchan);
+
 #ifdef __cplusplus
 }
 #endif

@@ -201,6 +201,7 @@ __global__ __launch_bounds__(WAVES * 64, 512 / (WAVES * 64)) void fdd_mfma16_k(
     static_assert(!BLK || (PIPE && MIRROR), "bin-block layout: pipelined form with mirror bins");
     constexpr int NT = WAVES * 64;        // threads
     constexpr int DPB = WAVES * MT * 16;  // DMs per workgroup
+    static_assert(DPB == DD_FDD_DM_BLOCK, "the DM block the host prices and splits by");
     constexpr int NDIR = MIRROR ? NS / 2 : NS;  // bins whose phasors are computed
     using G = Geo<PREC, NTL, NS, NT>;
     using PL = Planes<PREC>;

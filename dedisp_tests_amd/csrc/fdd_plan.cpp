@@ -155,11 +155,58 @@ size_t balanced_batch(size_t ndm, size_t most)
     most = std::max<size_t>(1, std::min(ndm, most));
     const size_t nbat = div_up(ndm, most);
     const size_t even = div_up(ndm, nbat);
-    const size_t blk = round_up(even, 256);
+    const size_t blk = round_up(even, DD_FDD_DM_BLOCK);
     return (blk <= most) ? blk : even;
 }
 
 }  // namespace
+
+// The supported length with the least estimated time.
+// Contraction: a chunk group of ntl 8-chunk tiles costs ntl tiles of products
+// plus the phasors, kPhasorTiles tiles' worth whatever its width (1024 ch x
+// 2048 DMs x 65536: one tile 20.9 ms, three 38.5 ms), for every bin, channel
+// and DM of a whole block (20 DMs cost as 256: priced by waves of 32 DMs, 1024
+// ch x 64701 samples x 20 DMs with delays to 22527 took 65536 and 3.11 ms in
+// float32 where 32768 takes 1.89; 256 DMs take 1.96).
+// Transforms: one per chunk and channel, one per chunk and DM.
+// The smallest volume of columns x bins leaves out phasors and transforms and
+// takes 131072 and one tile of 5 chunks at 1024 ch x 2^19 x 1000 DMs in
+// float32 (29.6 ms) where 65536 and two tiles of 11 take 18.3 ms, and at 8
+// beams x 15625 x 3000 DMs in bfloat16 65536 (36.4 ms) instead of 32768 (27.1
+// ms). The float16 form keeps the smallest volume: its rounding (2e-4 of the
+// result) depends on the segment length, and an output should not.
+extern "C" size_t dd_fdd_segment_length(int form, int prec, size_t dmax, const size_t* nsc, size_t n, size_t ndm,
+                                        size_t nchan)
+{
+    const Contraction kind = (Contraction)form;
+    ndm = std::max<size_t>(ndm, 1);
+    const double dms = (double)(kind == Contraction::VALU ? ndm : round_up(ndm, DD_FDD_DM_BLOCK));
+    size_t nfft = 0;
+    double best = -1;
+    for (size_t cand = 8192; cand <= 262144; cand *= 2) {
+        if (cand < dmax + 2 + 2) continue;
+        const size_t good = (cand - dmax) & ~size_t(1);
+        size_t chunks = 0;
+        for (size_t i = 0; i < n; ++i) chunks += div_up(nsc[i], good);
+        double columns = (double)chunks, tiles = columns / 8;  // computed chunk columns, padding included
+        if (kind == Contraction::MFMA32) {
+            columns = (double)round_up(chunks, 32);
+            tiles = columns / 8;
+        } else if (kind == Contraction::MFMA16) {
+            int ntl = 1;
+            size_t groups = 0;
+            dd_fdd_mfma16_tiles(chunks, prec, &ntl, &groups);
+            columns = (double)(groups * (size_t)ntl * 8);
+            tiles = (double)groups * ((double)ntl + kPhasorTiles);
+        }
+        double cost = kTile * tiles * (double)(cand / 2 + 1) * dms * (double)padded_channels(nchan) +
+                      (cand > 65536 ? kSplitTransform : kTransform) * (double)chunks * (double)cand *
+                          (double)(ndm + nchan);
+        if (prec == DEDISP_AMD_FDD_FP16) cost = columns * (double)(cand / 2 + 1);
+        if (best < 0 || cost < best) best = cost, nfft = cand;
+    }
+    return nfft;
+}
 
 FDDGPUPlan::FDDGPUPlan(size_type nchans, float_type dt, float_type f0, float_type df, int device_idx)
     : GPUPlan(nchans, dt, f0, df, device_idx), m_state(new FDDState)
@@ -368,55 +415,17 @@ void FDDGPUPlan::prepare_tables()
 }
 
 // Overlap-save segment length for series with nsc[0..n) outputs per DM: the
-// requested one, else the supported length (2^13 .. 2^18) with the least
-// estimated time. The reference instead doubles nfft from 16384 until a fifth
-// of it covers the maximum delay (src/fdd/FDDGPUPlan.cpp:756-762).
+// requested one, else dd_fdd_segment_length. The reference instead doubles
+// nfft from 16384 until a fifth of it covers the maximum delay
+// (src/fdd/FDDGPUPlan.cpp:756-762).
 size_t FDDGPUPlan::segment_length(const size_t* nsc, size_t n) const
 {
     const FDDState& st = *m_state;
     const size_t dmax = (size_t)st.dmax;
     size_t nfft = st.nfft_req;
-    if (!nfft) {
-        // Contraction: a chunk group of ntl 8-chunk tiles costs ntl tiles of
-        // products plus the phasors, kPhasorTiles tiles' worth whatever its
-        // width (1024 ch x 2048 DMs x 65536: one tile 20.9 ms, three 38.5 ms),
-        // for every bin, channel and DM.
-        // Transforms: one per chunk and channel, one per chunk and DM.
-        // The smallest volume of columns x bins, which this replaces, left out
-        // phasors and transforms and took 131072 and one tile of 5 chunks at
-        // 1024 ch x 2^19 x 1000 DMs in float32 (29.6 ms) where 65536 and two
-        // tiles of 11 take 18.3 ms, and at 8 beams x 15625 x 3000 DMs in
-        // bfloat16 65536 (36.4 ms) instead of 32768 (27.1 ms). The float16
-        // form keeps the smallest volume: its rounding (2e-4 of the result)
-        // depends on the segment length, and an output should not.
-        const Contraction kind = contraction_kind(st);
-        const double dms = (double)round_up(std::max<size_t>(m_dm_count, 1), 32);
-        double best = -1;
-        for (size_t cand = 8192; cand <= 262144; cand *= 2) {
-            if (cand < dmax + 2 + 2) continue;
-            const size_t good = (cand - dmax) & ~size_t(1);
-            size_t chunks = 0;
-            for (size_t i = 0; i < n; ++i) chunks += div_up(nsc[i], good);
-            double columns = (double)chunks, tiles = columns / 8;  // computed chunk columns, padding included
-            if (kind == Contraction::MFMA32) {
-                columns = (double)round_up(chunks, 32);
-                tiles = columns / 8;
-            } else if (kind == Contraction::MFMA16) {
-                int ntl = 1;
-                size_t groups = 0;
-                dd_fdd_mfma16_tiles(chunks, (int)st.precision, &ntl, &groups);
-                columns = (double)(groups * (size_t)ntl * 8);
-                tiles = (double)groups * ((double)ntl + kPhasorTiles);
-            }
-            double cost = kTile * tiles * (double)(cand / 2 + 1) * dms * (double)padded_channels(m_nchans) +
-                          (cand > 65536 ? kSplitTransform : kTransform) * (double)chunks * (double)cand *
-                              (dms + (double)m_nchans);
-            if (st.precision == DEDISP_AMD_FDD_FP16) cost = columns * (double)(cand / 2 + 1);
-            if (best < 0 || cost < best) best = cost, nfft = cand;
-        }
-        if (!nfft) DD_THROW(DEDISP_UNKNOWN_ERROR);  // max delay beyond the largest segment
-    }
-    if (nfft < dmax + 4) DD_THROW(DEDISP_UNKNOWN_ERROR);
+    if (!nfft)
+        nfft = dd_fdd_segment_length((int)contraction_kind(st), (int)st.precision, dmax, nsc, n, m_dm_count, m_nchans);
+    if (nfft < dmax + 4) DD_THROW(DEDISP_UNKNOWN_ERROR);  // max delay beyond the (largest) segment
     return nfft;
 }
 

@@ -1,0 +1,37 @@
+"""The automatic overlap-save segment length (dd_fdd_segment_length, host only)."""
+import ctypes as C
+
+import pytest
+
+FP32, BF16, FP16 = 0, 1, 2
+VALU, TILE32, TILE16 = 0, 1, 2
+LENGTHS = [8192, 16384, 32768, 65536, 131072, 262144]
+
+
+@pytest.fixture
+def segment_length(dd):
+    fn = dd.lib().dd_fdd_segment_length
+    fn.restype = C.c_size_t
+    fn.argtypes = [C.c_int, C.c_int, C.c_size_t, C.POINTER(C.c_size_t), C.c_size_t, C.c_size_t, C.c_size_t]
+
+    def call(form, prec, dmax, nsc, ndm, nchan):
+        return fn(form, prec, dmax, (C.c_size_t * len(nsc))(*nsc), len(nsc), ndm, nchan)
+
+    return call
+
+
+@pytest.mark.parametrize("ndm", [1, 16, 20, 32, 64, 200, 256])
+def test_few_trials_are_priced_as_a_whole_block(segment_length, ndm):
+    """The contraction computes 256 DMs whatever the list holds: at 1024
+    channels, 64701 samples and delays to 22527, 32768 takes 1.9 ms for 20 and
+    for 256 trials, 65536 3.1 ms."""
+    assert segment_length(TILE16, FP32, 22527, [64701 - 22527], ndm, 1024) == 32768
+
+
+@pytest.mark.parametrize("form", [VALU, TILE32, TILE16])
+@pytest.mark.parametrize("prec", [FP32, BF16, FP16])
+def test_length_holds_the_largest_delay(segment_length, form, prec):
+    for dmax in (0, 1, 8188, 8189, 65532, 65533, 262140):
+        n = segment_length(form, prec, dmax, [1, 50000, 0], 700, 512)
+        assert n in LENGTHS and n >= dmax + 4
+    assert segment_length(form, prec, 262141, [1000], 700, 512) == 0
