@@ -157,6 +157,15 @@ hipError_t dd_fdd_contract_mfma16(int prec, int mirror, const float2* X, size_t 
                                   float xscale, float2* Y, size_t Yp, const float2* ph_packed,
                                   const float* dmlist, const float* delay32, int cfg, int blocked,
                                   hipStream_t stream);
+// What the phasors of a chunk group cost dd_fdd_contract_mfma16, in 8-chunk
+// tiles of products, whatever the group's width (1024 ch x 2048 DMs x 65536,
+// float32: one tile 20.9 ms, three 38.5 ms). The tiles of a group and the
+// segment length are chosen by it; the tiles are the same for any value
+// between 1 and 2; of 90 series 6 take another length with 1.5 than with 1.3,
+// in 0.82 to 0.94 of the time in float32 (1000 ch x 5 beams x 252185 x 66 DMs
+// 19.6 -> 17.5 ms).
+#define DD_FDD_PHASOR_TILES 1.5
+
 // N-tiles (8 chunks each) per workgroup dd_fdd_contract_mfma16 uses for
 // nchunk chunks, and the number of chunk groups.
 int dd_fdd_mfma16_tiles(size_t nchunk, int prec, int* ntl, size_t* ngroups);

@@ -814,14 +814,14 @@ __global__ __launch_bounds__(WAVES * 64, 512 / (WAVES * 64)) void fdd_mfma16_k(
 extern "C" int dd_fdd_mfma16_tiles(size_t nchunk, int prec, int* ntl_out, size_t* ngroups_out)
 {
     // N-tiles per chunk group: fewest tiles plus the phasor cost of each group
-    // (every group regenerates the same phasors), about 1.5 tiles' worth
+    // (every group regenerates the same phasors)
     const int max_ntl = 3;
     (void)prec;
     double best = 1e300;
     int best_ntl = 1;
     for (int ntl = 1; ntl <= max_ntl; ++ntl) {
         const size_t groups = (nchunk + 8 * ntl - 1) / (8 * ntl);
-        const double cost = (double)(groups * ntl) + 1.5 * (double)groups;
+        const double cost = (double)(groups * ntl) + DD_FDD_PHASOR_TILES * (double)groups;
         if (cost < best || (cost == best && ntl > best_ntl)) best = cost, best_ntl = ntl;
     }
     if (ntl_out) *ntl_out = best_ntl;

@@ -109,7 +109,7 @@ constexpr size_t kZBudget = size_t(32) << 30;
 // Measured costs the segment length is chosen by (ns; 1024 ch x 2^20 samples):
 // the contraction of one tile of 8 chunks per bin, DM and channel, and the
 // transforms per sample of a chunk (on chip, and split beyond 65536).
-constexpr double kPhasorTiles = 1.3, kTile = 1.33e-4;
+constexpr double kTile = 1.33e-4;
 constexpr double kTransform = 2.3e-3, kSplitTransform = 4.3e-3;
 
 bool env_flag(const char* name)
@@ -163,11 +163,10 @@ size_t balanced_batch(size_t ndm, size_t most)
 
 // The supported length with the least estimated time.
 // Contraction: a chunk group of ntl 8-chunk tiles costs ntl tiles of products
-// plus the phasors, kPhasorTiles tiles' worth whatever its width (1024 ch x
-// 2048 DMs x 65536: one tile 20.9 ms, three 38.5 ms), for every bin, channel
-// and DM of a whole block (20 DMs cost as 256: priced by waves of 32 DMs, 1024
-// ch x 64701 samples x 20 DMs with delays to 22527 took 65536 and 3.11 ms in
-// float32 where 32768 takes 1.89; 256 DMs take 1.96).
+// plus the phasors (DD_FDD_PHASOR_TILES), for every bin, channel and DM of a
+// whole block (20 DMs cost as 256: priced by waves of 32 DMs, 1024 ch x 64701
+// samples x 20 DMs with delays to 22527 took 65536 and 3.11 ms in float32 where
+// 32768 takes 1.89; 256 DMs take 1.96).
 // Transforms: one per chunk and channel, one per chunk and DM.
 // The smallest volume of columns x bins leaves out phasors and transforms and
 // takes 131072 and one tile of 5 chunks at 1024 ch x 2^19 x 1000 DMs in
@@ -197,7 +196,7 @@ extern "C" size_t dd_fdd_segment_length(int form, int prec, size_t dmax, const s
             size_t groups = 0;
             dd_fdd_mfma16_tiles(chunks, prec, &ntl, &groups);
             columns = (double)(groups * (size_t)ntl * 8);
-            tiles = (double)groups * ((double)ntl + kPhasorTiles);
+            tiles = (double)groups * ((double)ntl + DD_FDD_PHASOR_TILES);
         }
         double cost = kTile * tiles * (double)(cand / 2 + 1) * dms * (double)padded_channels(nchan) +
                       (cand > 65536 ? kSplitTransform : kTransform) * (double)chunks * (double)cand *

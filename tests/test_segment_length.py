@@ -35,3 +35,14 @@ def test_length_holds_the_largest_delay(segment_length, form, prec):
         n = segment_length(form, prec, dmax, [1, 50000, 0], 700, 512)
         assert n in LENGTHS and n >= dmax + 4
     assert segment_length(form, prec, 262141, [1000], 700, 512) == 0
+
+
+@pytest.mark.parametrize("nchan,nsc,ndm,dmax,want", [
+    (64, [30770 - 3493] * 5, 78, 3493, 16384),     # 0.242 ms, 32768 0.294
+    (1000, [252185 - 60000] * 5, 66, 60000, 131072),  # 17.5 ms, 262144 19.6
+    (1024, [430837 - 12405], 373, 12405, 32768),   # 7.33 ms, 65536 7.81
+])
+def test_phasors_cost_what_the_tile_rule_says(segment_length, nchan, nsc, ndm, dmax, want):
+    """Lengths that turn on the phasors' cost: priced as where the tiles of a
+    chunk group are chosen, the faster of the two measured is taken."""
+    assert segment_length(TILE16, FP32, dmax, nsc, ndm, nchan) == want
