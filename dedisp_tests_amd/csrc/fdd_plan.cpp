@@ -161,7 +161,7 @@ size_t balanced_batch(size_t ndm, size_t most)
 
 }  // namespace
 
-// The supported length with the least estimated time.
+// float32: the supported length with the least estimated time.
 // Contraction: a chunk group of ntl 8-chunk tiles costs ntl tiles of products
 // plus the phasors (DD_FDD_PHASOR_TILES), for every bin, channel and DM of a
 // whole block (20 DMs cost as 256: priced by waves of 32 DMs, 1024 ch x 64701
@@ -169,11 +169,20 @@ size_t balanced_batch(size_t ndm, size_t most)
 // 32768 takes 1.89; 256 DMs take 1.96).
 // Transforms: one per chunk and channel, one per chunk and DM.
 // The smallest volume of columns x bins leaves out phasors and transforms and
-// takes 131072 and one tile of 5 chunks at 1024 ch x 2^19 x 1000 DMs in
-// float32 (29.6 ms) where 65536 and two tiles of 11 take 18.3 ms, and at 8
-// beams x 15625 x 3000 DMs in bfloat16 65536 (36.4 ms) instead of 32768 (27.1
-// ms). The float16 form keeps the smallest volume: its rounding (2e-4 of the
-// result) depends on the segment length, and an output should not.
+// takes 131072 and one tile of 5 chunks at 1024 ch x 2^19 x 1000 DMs (29.6 ms)
+// where 65536 and two tiles of 11 take 18.3 ms.
+//
+// bfloat16, float16: the smallest volume of chunk columns x bins, padding
+// included. A form's rounding is relative to the spectrum and spreads evenly
+// over the segment, so the error against float64 falls with the part of the
+// segment that holds data: bfloat16 2.98e-6 x sqrt(mean part), within 3 % from
+// 8192 to 262144. The least time takes segments with less padding (8 beams x
+// 15625 x 3000 DMs: 32768 and 27.1 ms instead of 65536 and 36.4), and with them
+// 2.95e-6 instead of 2.33e-6: accuracy that a caller may give up by setting the
+// segment length, not this rule. float32's error on hi + lo pairs is
+// below that of float32 products at whatever length either took (24 series
+// drawn from 32768 to 2^20 samples, streams and Fourier output among them:
+// 0.68 to 0.90 of it).
 extern "C" size_t dd_fdd_segment_length(int form, int prec, size_t dmax, const size_t* nsc, size_t n, size_t ndm,
                                         size_t nchan)
 {
@@ -201,7 +210,7 @@ extern "C" size_t dd_fdd_segment_length(int form, int prec, size_t dmax, const s
         double cost = kTile * tiles * (double)(cand / 2 + 1) * dms * (double)padded_channels(nchan) +
                       (cand > 65536 ? kSplitTransform : kTransform) * (double)chunks * (double)cand *
                           (double)(ndm + nchan);
-        if (prec == DEDISP_AMD_FDD_FP16) cost = columns * (double)(cand / 2 + 1);
+        if (prec != DEDISP_AMD_FDD_FP32) cost = columns * (double)(cand / 2 + 1);
         if (best < 0 || cost < best) best = cost, nfft = cand;
     }
     return nfft;

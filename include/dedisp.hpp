@@ -224,9 +224,8 @@ public:
     dedisp_amd_fdd_output get_output_mode() const;
     void set_precision(dedisp_amd_fdd_precision precision);
     dedisp_amd_fdd_precision get_precision() const;
-    /* nfft = 0 selects the supported segment length (2^13 .. 2^18) with the
-     * smallest contraction volume (dedisp_amd_fdd_set_segmented); segmented
-     * mode writes time series. */
+    /* nfft = 0 selects a supported segment length (2^13 .. 2^18) by the rule
+     * of dedisp_amd_fdd_set_segmented; segmented mode writes time series. */
     void set_segmented(int enable, dedisp_size nfft);
 
     /* Output length per DM, in floats, for nsamps input samples. */

@@ -69,10 +69,11 @@ dedisp_error dedisp_amd_fdd_set_output(dedisp_plan plan, dedisp_amd_fdd_output m
 dedisp_error dedisp_amd_fdd_set_precision(dedisp_plan plan, dedisp_amd_fdd_precision precision);
 /* enable=1 selects the time-segmented (overlap-save) path. nfft is the
  * segment length: a power of two from 2^13 to 2^18 larger than max_delay + 3,
- * or 0 for the supported length with the smallest contraction volume (chunk
- * columns of the contraction's tiles x (nfft/2 + 1)); the reference instead
- * doubles nfft from 16384 until
- * a fifth of it covers max_delay (src/fdd/FDDGPUPlan.cpp:756-762). The same
+ * or 0 for a supported length by rule: float32 the least estimated time,
+ * bfloat16 and float16 the smallest contraction volume (chunk columns of the
+ * contraction's tiles x (nfft/2 + 1)), since a shorter segment costs them
+ * accuracy; the reference instead doubles nfft from 16384 until a fifth of it
+ * covers max_delay (src/fdd/FDDGPUPlan.cpp:756-762). The same
  * choice picks the segments of the time-series and Fourier outputs when no
  * length is set, so any max_delay below 2^18 - 3 samples is supported. The
  * reference selects this path with the USE_SEGMENTED environment variable,
@@ -197,7 +198,7 @@ dedisp_error dedisp_amd_write_inf(const char* prefix, const dedisp_amd_fil_heade
  * beams; with DEDISP_DEVICE_POINTERS that sequence is captured in a HIP graph
  * and replayed while lengths, pointers, widths and DM list stay the same.
  * FDD plans writing time series use one segment length for the batch (the
- * set one, else the one with the smallest summed contraction volume) and run
+ * set one, else the one the same rule takes for all chunks together) and run
  * the overlap-save chunks of all beams through one forward transform, one
  * contraction and one inverse transform per group of beams; each beam's
  * output equals dedisp_execute on it alone with that segment length. Other

@@ -1,5 +1,6 @@
 """The automatic overlap-save segment length (dd_fdd_segment_length, host only)."""
 import ctypes as C
+import random
 
 import pytest
 
@@ -46,3 +47,32 @@ def test_phasors_cost_what_the_tile_rule_says(segment_length, nchan, nsc, ndm, d
     """Lengths that turn on the phasors' cost: priced as where the tiles of a
     chunk group are chosen, the faster of the two measured is taken."""
     assert segment_length(TILE16, FP32, dmax, nsc, ndm, nchan) == want
+
+
+def _smallest_volume(dmax, nsc):
+    """Chunk columns of the 16 x 16 tiles, padding included, times bins."""
+    best = None
+    for n in LENGTHS:
+        if n < dmax + 4:
+            continue
+        good = (n - dmax) & ~1
+        chunks = sum(-(-x // good) for x in nsc)
+        groups, ntl = min(((-(-chunks // (8 * t)), t) for t in (1, 2, 3)),
+                          key=lambda g: (g[0] * g[1] + 1.5 * g[0], -g[1]))
+        cost = 8 * groups * ntl * (n // 2 + 1)
+        if best is None or cost < best[0]:
+            best = cost, n
+    return best[1]
+
+
+@pytest.mark.parametrize("prec", [BF16, FP16])
+def test_reduced_precision_keeps_the_smallest_volume(segment_length, prec):
+    """A segment with less padding holds a larger error in these forms: the
+    estimated time, which takes such segments, is for float32 alone."""
+    assert segment_length(TILE16, prec, 24849, [15625] * 8, 3000, 1024) == 65536
+    assert segment_length(TILE16, FP32, 24849, [15625] * 8, 3000, 1024) == 32768
+    rng = random.Random(7)
+    for _ in range(400):
+        dmax = rng.randint(0, 100000)
+        nsc = [int(2 ** rng.uniform(10, 20)) for _ in range(rng.randint(1, 9))]
+        assert segment_length(TILE16, prec, dmax, nsc, rng.randint(1, 3000), 1024) == _smallest_volume(dmax, nsc)
