@@ -176,18 +176,7 @@ dd_tdd_tiling default_tiling(unsigned nbits)
     return packed_tiling(nbits);
 }
 
-// Whether ntiles time tiles x dm_count DMs are too few for the bit-plane
-// kernel, whose workgroups are larger (4096 outputs) and fewer: below about 96
-// of them the smaller ones of the other kernels keep more of the chip busy
-// (2-bit, 256 ch, 16 DMs a block: 48 workgroups 0.93 of the packed lanes'
-// speed, 112 1.34; 8-bit, 8 DMs a block and a gain of 1.2 at most: 384
-// workgroups, 1.5 a CU, 0.9, 1500 1.28).
 size_t planes_tiles(size_t nsc) { return div_up(nsc, size_t(32) * DD_TDD_PLANES_T); }
-bool too_few_for_planes(unsigned nbits, size_t ntiles, size_t dm_count)
-{
-    const dd_tdd_tiling t = default_tiling(nbits);
-    return ntiles * div_up(dm_count, (size_t)t.dms_per_wave * t.waves) < (nbits == 8 ? 448u : 96u);
-}
 
 constexpr size_t kLdsBudget = 64 * 1024;  // bytes of LDS per workgroup
 // LDS of a bit-plane workgroup: two per CU, or (1 DM per wave, sub-byte, for
@@ -197,6 +186,48 @@ constexpr size_t kLdsBudget = 64 * 1024;  // bytes of LDS per workgroup
 // packed lanes; 4-bit 1.07, 1.31, 1.31. 8-bit with one workgroup per CU lost to
 // the packed lanes, 2.60 against 2.16 ms.
 constexpr size_t kPlanesLds = 80 * 1024, kPlanesLdsOne = 158 * 1024;
+
+}  // namespace
+
+// The bit-plane kernel's workgroups are larger (4096 outputs) and fewer than
+// the other kernels', so they leave more of the chip idle where there are few.
+// 1- and 2-bit: from 96 of them on it is the faster one at any channel count
+// (96 to 560 workgroups, 16 to 256 ch: 1.2 to 3.3 times; 0.98 to 1.1 with two
+// tiles, the second half empty).
+// 4- and 8-bit gain less (1.7 and 1.4 times at most, 1024 ch) and lose it
+// where the channels are few or a last round of workgroups is nearly empty, so
+// both times are estimated: the planes' by rounds of 256 workgroups, two of
+// which share the CUs; the runs kernel's (4-bit) by its own rounds, three of
+// which do; the packed lanes' (8-bit) by the outputs. Fitted to 896 launches of
+// 16 to 1024 ch, 2 to 16 tiles and 96 to 2100 workgroups, within 6 % rms, and
+// taken with that to spare; below 48 ch the 4-bit estimates are too close to
+// each other to tell. Of those launches 4-bit takes 341 of 576, 8-bit 131 of
+// 320; a bound of 96 (8-bit: 448) workgroups took all of them and was slower by
+// more than 3 % on 122 and on 123, down to 0.67 (16 ch) and 0.71 (32 ch), where
+// these estimates are on 3 and on 3, down to 0.93 and 0.96. On 207 others drawn
+// at random the bound was slower on 35 of 143, the estimates on none of 79.
+extern "C" int dd_tdd_planes_pay(unsigned nbits, size_t nchans, size_t ntiles, size_t nout, size_t ndm)
+{
+    const dd_tdd_tiling t = default_tiling(nbits);
+    if (!dd_tdd_tiling_is_planes(t)) return 0;
+    const size_t dpb = (size_t)t.dms_per_wave * t.waves;
+    const size_t wgs = ntiles * div_up(ndm, dpb), rounds = div_up(wgs, size_t(256));
+    if (nbits <= 2) return wgs >= 96;
+    const double n = (double)nchans, out = (double)nout * (double)ndm * 1e-6;
+    if (nbits == 4) {  // us
+        const size_t runs = div_up(div_up(nout, size_t(7 * 256)) * div_up(ndm, size_t(16)), size_t(256));
+        const double part[3] = {0.0, 9.3 + 0.211 * n, 10.1 + 0.286 * n};
+        const double planes = 29.8 + 0.067 * n + 0.152 * out + (12.9 + 0.342 * n) * (double)(rounds / 2) +
+                              (7.7 + 0.215 * n) * (double)(rounds % 2);
+        const double other = 21.2 + 0.083 * n + 0.046 * out + (11.9 + 0.381 * n) * (double)(runs / 3) + part[runs % 3];
+        return nchans >= 48 && 1.04 * planes < other;
+    }
+    const double planes = 30.4 + (3.8 + 0.24 * n) * std::max((double)rounds, 1.4);
+    const double other = 21.4 + 0.147 * n + (0.459 + 0.0339 * n) * out;
+    return 1.06 * planes < other;
+}
+
+namespace {
 
 // Output samples per time tile of the channel-sum kernel: 7 runs of 256 for
 // the runs-layout kernel, 32 for the bit-plane kernel, 64 lanes x
@@ -697,7 +728,8 @@ void TDDPlan::execute_span(size_type nsamps, const byte_type* in, size_type in_n
 
     const unsigned nbits = (unsigned)in_nbits;
     prepare_tables(nbits, first_dm_idx, dm_count, true,
-                   !m_state->tuned[nbits].waves && too_few_for_planes(nbits, planes_tiles(nsc), dm_count));
+                   !m_state->tuned[nbits].waves &&
+                       !dd_tdd_planes_pay(nbits, m_nchans, planes_tiles(nsc), nsc, dm_count));
     st.row_words = row_words_for(nbits, nsamps, nsc);
 
     // ---- input ----
@@ -868,7 +900,8 @@ void TDDPlan::execute_noalloc(size_type nsamps, const byte_type* in, size_type i
     // bit-plane rows take whole tiles: where they do not fit, the packed-lane
     // layout (and its tables) may, and is kept for the series length
     const std::array<uint64_t, 3> packed_key = {m_tables_version, nbits, nsamps};
-    const bool few = !st.tuned[nbits].waves && too_few_for_planes(nbits, planes_tiles(nsc), m_dm_count);
+    const bool few = !st.tuned[nbits].waves &&
+                     !dd_tdd_planes_pay(nbits, m_nchans, planes_tiles(nsc), nsc, m_dm_count);
     if (few || st.noalloc_packed == packed_key) {
         if (!lay_out(true)) DD_THROW(DEDISP_MEM_ALLOC_FAILED);
     } else if (!lay_out(false)) {
@@ -945,10 +978,13 @@ void TDDPlan::execute_batch(size_type nbeams, const size_type* nsamps, const byt
     TDDState& st = *m_state;
     ctx.make_current();
     hipStream_t stream = ctx.exec;
-    size_t tiles = 0;
-    for (size_t b = 0; b < nbeams; ++b) tiles += planes_tiles(nsamps[b] - m_max_delay);
+    size_t tiles = 0, outputs = 0;
+    for (size_t b = 0; b < nbeams; ++b) {
+        tiles += planes_tiles(nsamps[b] - m_max_delay);
+        outputs += nsamps[b] - m_max_delay;
+    }
     prepare_tables(nbits, 0, m_dm_count, true,
-                   !st.tuned[nbits].waves && too_few_for_planes(nbits, tiles, m_dm_count));
+                   !st.tuned[nbits].waves && !dd_tdd_planes_pay(nbits, m_nchans, tiles, outputs, m_dm_count));
     if (!st.fast || st.nact == 0) {
         // weighted killmask or 16/32-bit samples: one beam after another
         for (size_t b = 0; b < nbeams; ++b)

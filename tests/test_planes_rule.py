@@ -1,0 +1,42 @@
+"""Which launches the bit-plane channel sum takes (dd_tdd_planes_pay, host only)."""
+import ctypes as C
+
+import pytest
+
+
+@pytest.fixture
+def pays(dd):
+    fn = dd.lib().dd_tdd_planes_pay
+    fn.restype = C.c_int
+    fn.argtypes = [C.c_uint] + [C.c_size_t] * 4
+    return lambda nbits, nch, nout, ndm: bool(fn(nbits, nch, -(-nout // 4096), nout, ndm))
+
+
+# times on the other kernels and on bit planes (us)
+@pytest.mark.parametrize("nbits,nch,nout,ndm,other,planes", [
+    (4, 16, 6144, 2560, 41, 61), (4, 32, 8192, 1536, 44, 58), (4, 64, 6554, 1024, 62.2, 69.5),
+    (4, 16, 98559, 1454, 208, 284), (4, 32, 7877, 13432, 180, 208),
+    (4, 64, 9600, 1024, 66.5, 70.4), (4, 64, 26214, 256, 63.8, 69.1), (4, 64, 6144, 2560, 64, 80),
+    (8, 32, 6144, 2080, 49, 69), (8, 64, 8192 * 4, 520, 74, 87), (8, 64, 6144, 4096, 116, 144),
+    (8, 256, 6144, 2080, 186, 237), (8, 256, 9600, 1024, 160.4, 173.7), (8, 1024, 6144, 2080, 709, 806),
+])
+def test_launches_that_bit_planes_slow_down_stay_off_them(pays, nbits, nch, nout, ndm, other, planes):
+    assert other < planes and not pays(nbits, nch, nout, ndm)
+
+
+@pytest.mark.parametrize("nbits,nch,nout,ndm,other,planes", [
+    (4, 64, 65536, 448, 90, 69), (4, 256, 65536, 384, 311, 209), (4, 1024, 32768, 384, 416, 329),
+    (4, 1024, 999178, 1167, 22900, 14600), (8, 256, 32768, 1024, 346, 289),
+    (8, 1024, 15625, 3000, 1920, 1430), (8, 1024, 26214, 256, 447.3, 371.5), (8, 1024, 65536, 1024, 2521, 1946),
+    (2, 64, 8192, 768, 72, 49), (2, 512, 4 * 600000, 1024, 21800, 8300), (1, 64, 6144, 1024, 74, 43),
+    (1, 512, 176150, 501, 990, 350),
+])
+def test_launches_that_bit_planes_speed_up_take_them(pays, nbits, nch, nout, ndm, other, planes):
+    assert planes < other and pays(nbits, nch, nout, ndm)
+
+
+@pytest.mark.parametrize("nbits", [1, 2, 4, 8, 16, 32])
+def test_smallest_launches_and_wide_samples(pays, nbits):
+    assert not pays(nbits, 64, 1, 1) and not pays(nbits, 1024, 4096, 16)
+    if nbits > 8:
+        assert not pays(nbits, 1024, 1 << 20, 2048)
