@@ -122,8 +122,8 @@ bool env_flag(const char* name)
 // with re/im along N, float32 as float16 hi + lo pairs (1024 ch x 2048 DMs x
 // 23 chunks of 65536: 39.7 ms against 120 ms on float32 matrix products, and
 // nearer the float64 result). DEDISP_FDD_MFMA32=1 selects the 32 x 32 tile
-// kernel instead (DEDISP_FDD_FP32_TILE16=1 keeps float32 on 16 x 16 tiles),
-// and DEDISP_FDD_VALU=1 the float32 vector-ALU form.
+// kernel instead (float32: float32 products), and DEDISP_FDD_VALU=1 the
+// float32 vector-ALU form.
 // The autotuner's choices (FDDGPUPlan::autotune) replace these defaults for
 // the precision they were timed with; the environment variables override both.
 enum class Contraction { VALU, MFMA32, MFMA16 };
@@ -134,10 +134,7 @@ bool tuned(const FDDState& st) { return st.tuned_prec == (int)st.precision; }
 Contraction contraction_kind(const FDDState& st)
 {
     const bool t = tuned(st) && st.tuned_form >= 0;
-    if (st.precision == DEDISP_AMD_FDD_FP32) {
-        if (env_flag("DEDISP_FDD_VALU")) return Contraction::VALU;
-        if (env_flag("DEDISP_FDD_FP32_TILE16")) return Contraction::MFMA16;
-    }
+    if (st.precision == DEDISP_AMD_FDD_FP32 && env_flag("DEDISP_FDD_VALU")) return Contraction::VALU;
     if (env_flag("DEDISP_FDD_MFMA32")) return Contraction::MFMA32;
     return (t && st.tuned_form == 3) ? Contraction::MFMA32 : Contraction::MFMA16;
 }

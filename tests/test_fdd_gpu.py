@@ -533,3 +533,32 @@ def test_fdd_waves_past_the_last_dm(dd, orc, prec, ndm):
     assert rel_l2(out, ref) < PREC_TOL[prec]
     assert rel_l2(out[-1], ref[-1]) < PREC_TOL[prec]
     plan.close()
+
+
+@pytest.mark.parametrize("nbits", [1, 8])
+@pytest.mark.parametrize("nchunk,ndm", [(1, 70), (31, 257), (32, 1), (33, 256)])
+def test_fdd_fp32_products_on_32x32_tiles(dd, orc, monkeypatch, nchunk, ndm, nbits):
+    """Float32 products (DEDISP_FDD_MFMA32=1) against the oracle, around their
+    tiles of 32 chunks and 256 DMs, whatever the variable that once kept float32
+    on 16 x 16 tiles says: one rounding of 2^-24 per stage of the two
+    transforms, and per channel, in quadrature, of the two sums a result is
+    made of. Another arithmetic than the default's, so not its bits."""
+    nch, dt, f0, df = 104, 64e-6, 1581.8, -1.0
+    dms = np.linspace(0, 150, ndm, dtype=f32) if ndm > 1 else np.array([150], dtype=f32)
+    rng = np.random.default_rng(nchunk + nbits)
+    outs = []
+    for tiles32 in ("1", "0"):
+        monkeypatch.setenv("DEDISP_FDD_MFMA32", tiles32)
+        monkeypatch.setenv("DEDISP_FDD_FP32_TILE16", "1")
+        plan = _fdd_plan(dd, nch, dt, f0, df, nfft=8192, prec=dd.FDD_FP32)
+        plan.set_dm_list(dms)
+        if not outs:
+            good = (8192 - plan.max_delay) & ~1
+            nsamps = plan.max_delay + nchunk * good - good // 3
+            s = rng.integers(0, 1 << nbits, size=(nsamps, nch)).astype(np.uint8)
+            delays = orc.delay_table(nch, f32(dt), f32(f0), f32(df))
+            ref = orc.fdd_timeseries(nch, delays, dms, nsamps, plan.max_delay, s, nbits=nbits)
+        outs.append(plan.execute(dd.pack_samples(s, nbits), nbits, 32))
+        plan.close()
+    assert rel_l2(outs[0], ref) < (2 * 13 + 2 * np.sqrt(nch)) * 2.0**-24
+    assert not np.array_equal(outs[0], outs[1])
