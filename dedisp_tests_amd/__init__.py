@@ -111,6 +111,7 @@ _SIG = [
     ("dedisp_amd_execute_batch", C.c_int, [C.c_void_p, C.c_ulong, C.POINTER(C.c_ulong), C.POINTER(C.c_void_p),
                                            C.c_ulong, C.POINTER(C.c_void_p), C.c_ulong, C.c_uint]),
     ("dedisp_amd_autotune", C.c_int, [C.c_void_p, C.c_ulong, C.c_ulong, C.c_ulong, C.c_void_p]),
+    ("dedisp_amd_get_channel_sum", C.c_int, [C.c_void_p, C.c_void_p]),
     ("dedisp_amd_execute_noalloc", C.c_int,
      [C.c_void_p, C.c_ulong, C.c_void_p, C.c_ulong, C.c_void_p, C.c_ulong, C.c_uint]),
     ("dedisp_select_implementation", C.c_int, [C.c_int]),
@@ -400,6 +401,12 @@ class Plan:
         t = Tuning()
         _check(lib().dedisp_amd_autotune(self._h, nsamps, in_nbits, out_nbits, C.byref(t)), "dedisp_amd_autotune")
         return t.as_dict()
+
+    def channel_sum(self) -> dict:
+        """Tiling of the channel-sum kernel the last execute ran (dedisp_amd_get_channel_sum)."""
+        t = Tuning()
+        _check(lib().dedisp_amd_get_channel_sum(self._h, C.byref(t)), "dedisp_amd_get_channel_sum")
+        return {k: getattr(t, k) for k in ("samples_per_lane", "dms_per_wave", "waves", "chunk_channels")}
 
 
 def pack_samples(samples: np.ndarray, nbits: int) -> np.ndarray:

@@ -313,6 +313,14 @@ dedisp_error dedisp_amd_autotune(dedisp_plan plan, dedisp_size nsamps, dedisp_si
     return DEDISP_INVALID_PLAN;
 }
 
+dedisp_error dedisp_amd_get_channel_sum(const dedisp_plan plan, dedisp_amd_tuning* result)
+{
+    if (!plan) return DEDISP_INVALID_PLAN;
+    if (!result) return DEDISP_INVALID_POINTER;
+    if (dedisp::TDDPlan* t = as_tdd(plan)) return guarded([&] { t->get_channel_sum(result); });
+    return DEDISP_INVALID_PLAN;
+}
+
 dedisp_error dedisp_sync(void)
 {
     if (hipDeviceSynchronize() != hipSuccess) {

@@ -1140,6 +1140,17 @@ void TDDPlan::execute_batch(size_type nbeams, const size_type* nsamps, const byt
     }
 }
 
+void TDDPlan::get_channel_sum(dedisp_amd_tuning* shape) const
+{
+    const TDDState& st = *m_state;
+    *shape = dedisp_amd_tuning{};
+    if (!st.fast) return;
+    shape->samples_per_lane = st.tiling.samples_per_lane;
+    shape->dms_per_wave = st.tiling.dms_per_wave;
+    shape->waves = st.tiling.waves;
+    shape->chunk_channels = st.tiling.chunk_channels;
+}
+
 double TDDPlan::autotune(size_type nsamps, size_type in_nbits, size_type out_nbits,
                          dedisp_amd_tuning* chosen)
 {

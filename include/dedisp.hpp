@@ -169,6 +169,10 @@ public:
     double autotune(size_type nsamps, size_type in_nbits, size_type out_nbits,
                     dedisp_amd_tuning* chosen);
 
+    /* Tiling of the channel-sum kernel the last execute ran
+     * (dedisp_amd_get_channel_sum). */
+    void get_channel_sum(dedisp_amd_tuning* shape) const;
+
     /* execute() on device pointers with every device buffer it needs (the
      * transposed input rows and the delay tables) carved out of the caller's
      * scratch of scratch_bytes, allocating no device memory

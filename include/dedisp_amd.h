@@ -237,6 +237,11 @@ typedef struct {
 dedisp_error dedisp_amd_autotune(dedisp_plan plan, dedisp_size nsamps, dedisp_size in_nbits,
                                  dedisp_size out_nbits, dedisp_amd_tuning* result);
 
+/* The tiling of the channel-sum kernel that the last execute of a TDD or legacy
+ * plan ran (samples_per_lane 64: bit planes; 28 with 4-bit input: the runs
+ * layout; all 0: the generic kernel, or none yet); the other fields are 0. */
+dedisp_error dedisp_amd_get_channel_sum(const dedisp_plan plan, dedisp_amd_tuning* result);
+
 /* ---------------------------------------------------------------------------
  * Allocation-free execution. No counterpart in the reference: for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving

@@ -570,3 +570,111 @@ def test_tdd_planes_noalloc_at_the_scratch_limit(dd):
         torch.cuda.synchronize()
         assert torch.equal(a, b), n
     plan.close()
+
+
+def _shape(plan):
+    c = plan.channel_sum()
+    return c["samples_per_lane"], c["dms_per_wave"], c["waves"]
+
+
+@pytest.mark.parametrize("nbits,step,dms_per_wave", [
+    *[(b, s, w) for b in (1, 2, 4) for s, w in ((66, 2), (75, 1), (330, 1), (340, 0))], (8, 60, 1), (8, 66, 0)])
+def test_tdd_planes_windows_at_the_lds_limits(dd, orc, monkeypatch, nbits, step, dms_per_wave):
+    """Delays up to step samples apart from DM to DM, on each side of the LDS of
+    two workgroups per CU (2 DMs per wave up to 70 samples, 8-bit 1 DM up to 60)
+    and of one (1 DM per wave up to 330); 0: too wide for bit planes. Single
+    executes and a batch, whose launch with more than 64 KB is captured."""
+    import torch
+    monkeypatch.setenv("DEDISP_TDD_TILING", "64,1,8,16" if nbits == 8 else "64,2,8,16")
+    nch, nout, geom = 40, 4500, (64e-6, 1500.0, -10.0)
+    plan = dd.Plan(nch, *geom, impl=dd.TDD)
+    delays = orc.delay_table(nch, *[f32(g) for g in geom])
+    dms = (np.arange(33) * (step / float(delays[-1]))).astype(f32)
+    plan.set_dm_list(dms)
+    md = plan.max_delay
+    rng = np.random.default_rng(step + nbits)
+    data = [dd.pack_samples(rng.integers(0, 1 << nbits, size=(n + md, nch)).astype(np.uint8), nbits) for n in (nout, 300)]
+    ref = [orc.tdd(nch, delays, None, dms, len(d), md, d, nbits, 32) for d in data]
+    assert np.array_equal(plan.execute(data[0], nbits, 32), ref[0])
+    want = (64, dms_per_wave, 8)
+    assert _shape(plan) == want if dms_per_wave else _shape(plan)[0] != 64
+    d_in = [torch.from_numpy(d).cuda() for d in data]
+    d_out = [torch.empty(r.shape, dtype=torch.float32, device="cuda") for r in ref]
+    for _ in range(3):
+        for o in d_out:
+            o.zero_()
+        torch.cuda.synchronize()
+        assert plan.execute_batch_raw([len(d) for d in data], d_in, nbits, d_out, 32, dd.DEVICE_POINTERS) == 0
+        torch.cuda.synchronize()
+        assert all(np.array_equal(o.cpu().numpy(), r) for o, r in zip(d_out, ref))
+    plan.close()
+
+
+@pytest.mark.parametrize("nbits,shape", PLANES_SHAPES)
+@pytest.mark.parametrize("start", [20224, 20288, 20289, 20352, 20479, 20480])
+def test_tdd_planes_windows_far_into_the_series(dd, orc, monkeypatch, nbits, shape, start):
+    """Trials close together at a high DM: windows that start several tiles
+    after the outputs (the last channel's at start) and whose runs end just
+    before the next tile's (20224, 20288: run 30 or 30 and a half on, two runs)
+    or just after it; killed channels."""
+    monkeypatch.setenv("DEDISP_TDD_TILING", f"64,{shape},16")
+    nch, geom = 72, (64e-6, 1500.0, -400.0 / 72)
+    delays = orc.delay_table(nch, *[f32(g) for g in geom])
+    dms = ((start + np.arange(24) * 2.5) / float(delays[-1])).astype(f32)
+    lo = np.rint(dms[0] * delays).astype(int)
+    assert lo[-1] == start and len({int(x) // 4096 for x in lo}) >= 5
+    runs = lo // 128 % 32 + (lo % 128 + 192 + 127) // 128
+    assert (runs > 32).any() and (runs <= 32).any()
+    assert (runs[-1] > 32) == (start in (20289, 20352, 20479))
+    km = np.ones(nch, np.int32)
+    km[3::7] = 0
+    plan = dd.Plan(nch, *geom, impl=dd.TDD)
+    plan.set_dm_list(dms)
+    plan.set_killmask(km)
+    s = np.random.default_rng(start + nbits).integers(0, 1 << nbits, size=(4100 + plan.max_delay, nch)).astype(np.uint8)
+    data = dd.pack_samples(s, nbits)
+    out = plan.execute(data, nbits, 32)
+    w = shape.split(",")
+    assert _shape(plan) == (64, int(w[0]), int(w[1]))
+    assert np.array_equal(out, orc.tdd(nch, delays, km, dms, len(s), plan.max_delay, data, nbits, 32))
+    plan.close()
+
+
+def test_tdd_planes_host_outputs_in_dm_blocks(dd):
+    """Host outputs of more than 256 MB come in blocks of DMs, each a launch
+    with its own part of the tables: the same as one launch on device pointers."""
+    import torch
+    nch, nbits, ndm, nout = 32, 2, 160, 600_000
+    plan = dd.Plan(nch, 64e-6, 1500.0, -12.5, impl=dd.TDD)
+    plan.set_dm_list(np.linspace(0, 200, ndm, dtype=f32))
+    n = nout + plan.max_delay
+    d_in = torch.randint(0, 256, (n, nch * nbits // 8), dtype=torch.uint8, device="cuda")
+    d_out = torch.empty((ndm, nout), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    assert plan.execute_raw(n, d_in, nbits, d_out, 32, dd.DEVICE_POINTERS) == 0
+    assert _shape(plan)[0] == 64
+    torch.cuda.synchronize()
+    assert np.array_equal(plan.execute(d_in.cpu().numpy(), nbits, 32), d_out.cpu().numpy())
+    plan.close()
+
+
+@pytest.mark.parametrize("nbits,nch,short,long", [(1, 40, 1500, 24000), (2, 40, 1500, 24000), (4, 64, 6554, 26214),
+                                                  (8, 256, 6144, 32768)])
+def test_tdd_default_kernel_on_each_side_of_the_rule(dd, orc, nbits, nch, short, long):
+    """Whichever kernel the size takes, one plan's outputs are the oracle's,
+    and the size does take one and the other (dd_tdd_planes_pay)."""
+    geom = (64e-6, 1500.0, -400.0 / nch)
+    plan = _plan(dd, nch, *geom)
+    dms = np.linspace(0, 40, 1024, dtype=f32)
+    plan.set_dm_list(dms)
+    delays = orc.delay_table(nch, *[f32(g) for g in geom])
+    rng = np.random.default_rng(nbits)
+    md, rows = plan.max_delay, [0, 511, 1023]
+    for nout, planes in ((long, True), (short, False), (long, True)):
+        s = rng.integers(0, 1 << nbits, size=(md + nout, nch)).astype(np.uint8)
+        data = dd.pack_samples(s, nbits)
+        out = plan.execute(data, nbits, 32)
+        assert (_shape(plan)[0] == 64) == planes, nout
+        ref = [orc.tdd(nch, delays, None, dms, len(s), md, data, nbits, 32, first_dm=i, dm_count=1)[0] for i in rows]
+        assert np.array_equal(out[rows], np.array(ref)), nout
+    plan.close()
