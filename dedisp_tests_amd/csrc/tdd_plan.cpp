@@ -1162,14 +1162,16 @@ double TDDPlan::autotune(size_type nsamps, size_type in_nbits, size_type out_nbi
     GPUContext& ctx = *m_ctx;
     TDDState& st = *m_state;
     ctx.make_current();
-    // every instantiated shape with 16- and 32-channel staging chunks
+    // every instantiated shape, with 16- and 32-channel staging chunks but for
+    // bit planes, whose chunks the width sets
     dd_tdd_tiling cand[128];
     const int nshape = std::min(dd_tdd_lds_tilings(nbits, cand, 64), 64);
+    int ncand = nshape;
     for (int i = 0; i < nshape; ++i) {
-        cand[nshape + i] = cand[i];
-        cand[nshape + i].chunk_channels = 32;
+        if (dd_tdd_tiling_is_planes(cand[i])) continue;
+        cand[ncand] = cand[i];
+        cand[ncand++].chunk_channels = 32;
     }
-    const int ncand = 2 * nshape;
     const size_t row_bytes = (m_nchans * nbits + 7) / 8;
     const size_t nsc = nsamps - m_max_delay, out_bytes = out_nbits / 8;
     DeviceBuffer d_in, d_out;
@@ -1181,7 +1183,7 @@ double TDDPlan::autotune(size_type nsamps, size_type in_nbits, size_type out_nbi
     DD_HIP(hipEventCreate(&e1));
     const dd_tdd_tiling saved = st.tuned[nbits];
     double best = -1;
-    dd_tdd_tiling best_t{};
+    dd_tdd_tiling best_t{}, best_ran{};
     int timed = 0;
     try {
         for (int i = 0; i < ncand; ++i) {
@@ -1190,8 +1192,13 @@ double TDDPlan::autotune(size_type nsamps, size_type in_nbits, size_type out_nbi
                 execute_guru(nsamps, d_in.as<uint8_t>(), in_nbits, row_bytes, d_out.as<uint8_t>(), out_nbits,
                              nsc * out_bytes, 0, m_dm_count, DEDISP_DEVICE_POINTERS);
             };
-            run();  // builds the tables for this tiling
-            if (!st.fast) break;  // weighted killmask: nothing to choose
+            // another kernel runs where the candidate's windows do not fit, and
+            // for a weighted killmask
+            prepare_tables(nbits, 0, m_dm_count, /*upload=*/false);
+            if (!st.fast || st.tiling.samples_per_lane != cand[i].samples_per_lane ||
+                st.tiling.dms_per_wave != cand[i].dms_per_wave || st.tiling.waves != cand[i].waves)
+                continue;
+            run();
             DD_HIP(hipEventRecord(e0, ctx.exec));
             run();
             DD_HIP(hipEventRecord(e1, ctx.exec));
@@ -1199,7 +1206,7 @@ double TDDPlan::autotune(size_type nsamps, size_type in_nbits, size_type out_nbi
             float ms = 0.f;
             DD_HIP(hipEventElapsedTime(&ms, e0, e1));
             ++timed;
-            if (best < 0 || ms < best) best = ms, best_t = cand[i];
+            if (best < 0 || ms < best) best = ms, best_t = cand[i], best_ran = st.tiling;
         }
     } catch (...) {
         st.tuned[nbits] = saved;
@@ -1211,7 +1218,7 @@ double TDDPlan::autotune(size_type nsamps, size_type in_nbits, size_type out_nbi
     (void)hipEventDestroy(e1);
     st.tuned[nbits] = (best >= 0) ? best_t : saved;
     if (chosen) {
-        const dd_tdd_tiling t = (best >= 0) ? best_t : default_tiling(nbits);
+        const dd_tdd_tiling t = (best >= 0) ? best_ran : default_tiling(nbits);
         *chosen = dedisp_amd_tuning{};
         chosen->samples_per_lane = t.samples_per_lane;
         chosen->dms_per_wave = t.dms_per_wave;

@@ -328,3 +328,24 @@ def test_fdd_batch_graph_replays(dd):
         torch.cuda.synchronize()
         for i in range(len(lengths)):
             assert torch.equal(d_out[i], one[i]), (rep, i)
+
+
+@pytest.mark.parametrize("nbits,step", [(1, 20), (1, 100), (2, 400), (4, 20), (4, 100), (4, 400), (8, 30), (8, 100)])
+def test_autotune_reports_the_tiling_that_runs(dd, orc, nbits, step):
+    """Delays up to step samples apart from DM to DM: shapes whose windows do not
+    fit run another kernel, whose time is not theirs. What the autotuner reports
+    is what the next execute runs."""
+    nch, geom = 64, (64e-6, 1500.0, -6.25)
+    plan = dd.Plan(nch, *geom, impl=dd.TDD)
+    delays = orc.delay_table(nch, *[f32(g) for g in geom])
+    dms = (np.arange(64) * (step / float(delays[-1]))).astype(f32)
+    plan.set_dm_list(dms)
+    n = plan.max_delay + 9000
+    r = plan.autotune(n, nbits, 32)
+    rng = np.random.default_rng(step)
+    data = _packed(dd, rng, n, nch, nbits)
+    out = plan.execute(data, nbits, 32)
+    assert plan.channel_sum() == {k: r[k] for k in ("samples_per_lane", "dms_per_wave", "waves", "chunk_channels")}
+    assert r["best_ms"] > 0 and r["candidates"] >= 2
+    assert np.array_equal(out, orc.tdd(nch, delays, None, dms, n, plan.max_delay, data, nbits, 32))
+    plan.close()
