@@ -289,3 +289,43 @@ def test_quotient_from_the_reciprocal(vmax, out_range):
         r = (num.astype(np.float64) - q.astype(np.float64) * np.float64(den)).astype(np.float32)
         got = (q.astype(np.longdouble) + r.astype(np.longdouble) * np.longdouble(rcp)).astype(np.float32)
         assert np.array_equal(got, num / den), nch
+
+
+QUOTIENT = r'''
+#include <atomic>
+#include <cmath>
+#include <cstdio>
+#include <thread>
+#include <vector>
+int main()
+{
+    std::atomic<int> next{1}, bad{0};
+    auto work = [&] {
+        for (int nch; (nch = next++) <= 8192;)
+            for (int vmax : {1, 3, 15, 255})
+                for (float range : {1.f, 255.f, 65535.f}) {
+                    const float den = (float)(vmax * nch), rcp = 1.0f / den;
+                    int wrong = 0;
+                    for (int s = 0; s <= vmax * nch; ++s) {
+                        const float num = (float)s * range, q = num * rcp;
+                        wrong += std::fma(std::fma(-q, den, num), rcp, q) != num / den;
+                    }
+                    if (wrong) std::printf("%d channels of %d, range %g: %d\n", nch, vmax, range, wrong), bad = 1;
+                }
+    };
+    std::vector<std::thread> t;
+    for (unsigned i = 0; i < 4; ++i) t.emplace_back(work);
+    for (auto& x : t) x.join();
+    return bad;
+}
+'''
+
+
+def test_quotient_from_the_reciprocal_of_every_sum(tmp_path):
+    """The same for every sum of every channel count up to the TDD limit of 8192."""
+    import subprocess
+    (tmp_path / "quotient.cpp").write_text(QUOTIENT)
+    subprocess.run(["g++", "-O3", "-march=native", "-ffp-contract=off", "-pthread", "-std=c++17",
+                    str(tmp_path / "quotient.cpp"), "-o", str(tmp_path / "quotient")], check=True, timeout=120)
+    r = subprocess.run([str(tmp_path / "quotient")], capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stdout
