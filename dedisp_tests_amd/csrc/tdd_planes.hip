@@ -105,9 +105,11 @@ __global__ __launch_bounds__(256) void tdd_transpose_planes_k(
     const bool words = ((in_stride | reinterpret_cast<uintptr_t>(in)) & 3u) == 0;
     const int w = tid % TP_W, row0 = tid / TP_W;
     const size_t b = b0 + 4 * (size_t)w;
-    if (words && row_bytes % 4 == 0 && tq + 31 * T + TP_P <= nsamps) {
+    if (words && (row_bytes % 4 == 0 || b0 + TP_W * 4 <= row_bytes) && tq + 31 * T + TP_P <= nsamps) {
         // whole words of whole rows: a thread's word lies in the row or beyond
-        // it (zeros); 16 loads are issued before the first is waited on
+        // it (zeros); 16 loads are issued before the first is waited on (rows
+        // of odd bytes in a padded stride, in all but the last tile: 4108 2-bit
+        // channels, stride 1028, 200000 samples 154 us, guarded throughout 282)
         for (int n0 = 0; n0 < 64; n0 += 16) {
             uint32_t v[16];
 #pragma unroll

@@ -678,3 +678,32 @@ def test_tdd_default_kernel_on_each_side_of_the_rule(dd, orc, nbits, nch, short,
         ref = [orc.tdd(nch, delays, None, dms, len(s), md, data, nbits, 32, first_dm=i, dm_count=1)[0] for i in rows]
         assert np.array_equal(out[rows], np.array(ref)), nout
     plan.close()
+
+
+@pytest.mark.parametrize("planes", [False, True])
+@pytest.mark.parametrize("nbits,nch", [(8, 131), (8, 259), (4, 262), (4, 518), (2, 524), (2, 1036), (1, 1048)])
+def test_tdd_rows_of_odd_bytes_in_a_padded_stride(dd, orc, monkeypatch, nbits, nch, planes):
+    """Rows of 131 or 259 bytes 4 bytes apart from a multiple of 128: whole
+    words up to the last one, whose padding (all ones) must not be read."""
+    import torch
+    packed = {1: "32,2,4,16", 2: "16,2,4,16", 4: "28,4,4,32", 8: "16,2,4,16"}[nbits]
+    monkeypatch.setenv("DEDISP_TDD_TILING", packed if not planes else "64,1,8,16" if nbits == 8 else "64,2,8,16")
+    geom = (64e-6, 1500.0, -400.0 / nch)
+    plan = dd.Plan(nch, *geom, impl=dd.TDD)
+    dms = np.linspace(0, 10, 20, dtype=f32)
+    plan.set_dm_list(dms)
+    md, rng = plan.max_delay, np.random.default_rng(nch + nbits)
+    n = md + 8300
+    s = rng.integers(0, 1 << nbits, size=(n, nch)).astype(np.uint8)
+    data = dd.pack_samples(s, nbits)
+    stride = (data.shape[1] + 3) // 4 * 4 + 4
+    padded = torch.full((n, stride), 255, dtype=torch.uint8, device="cuda")
+    padded[:, : data.shape[1]] = torch.from_numpy(data).cuda()
+    out = torch.empty((len(dms), n - md), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    assert plan.execute_adv(n, padded, nbits, stride, out, 32, (n - md) * 4, dd.DEVICE_POINTERS) == 0
+    assert (_shape(plan)[0] == 64) == planes
+    torch.cuda.synchronize()
+    delays = orc.delay_table(nch, *[f32(g) for g in geom])
+    assert np.array_equal(out.cpu().numpy(), orc.tdd(nch, delays, None, dms, n, md, data, nbits, 32))
+    plan.close()
