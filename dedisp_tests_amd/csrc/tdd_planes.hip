@@ -393,11 +393,12 @@ __global__ __launch_bounds__(WAVES * 64, 4) void tdd_planes_k(
         for (int n = 0; n < IPW; ++n) {
             const uint32_t item = item_of(n);
             const uint32_t a = d[n].x, p = 64 * (item % G) + lane;
+            const uint32_t first = planes_lds_first(item / G, stride, a, p, NB);
             planes_stage(a, P, p, [&](int k, uint32_t shift, uint32_t u, bool in) {
                 uint32_t v[NB];
 #pragma unroll
                 for (int b = 0; b < NB; ++b) v[b] = __builtin_amdgcn_alignbit(w[n][k + 1][b], w[n][k][b], shift);
-                if (in) write_planes<NB>(lds + planes_lds_word(item / G, stride, planes_window_pos(a, p, u), NB), v);
+                if (in) write_planes<NB>(lds + planes_lds_word(first, u, NB), v);
             });
         }
     };

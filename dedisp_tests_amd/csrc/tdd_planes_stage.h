@@ -22,12 +22,17 @@ DD_STAGE_FN uint32_t planes_window_pos(uint32_t a, uint32_t p, uint32_t u)
     return p - a % DD_TDD_PLANES_T + u * DD_TDD_PLANES_T;
 }
 
-// LDS word of that position in the window of slot, windows of stride positions
-// of nbits words. The whole sum stays a 32-bit unsigned (a position before the
-// window wraps, and is not written), so no address outside LDS is ever formed.
-DD_STAGE_FN uint32_t planes_lds_word(uint32_t slot, uint32_t stride, uint32_t pos, uint32_t nbits)
+// LDS word of a lane's first word in the window of slot, windows of stride
+// positions of nbits words, and of its word u from that. The whole sum stays a
+// 32-bit unsigned (a first word before the window wraps, and is not written),
+// so no address outside LDS is ever formed.
+DD_STAGE_FN uint32_t planes_lds_first(uint32_t slot, uint32_t stride, uint32_t a, uint32_t p, uint32_t nbits)
 {
-    return (slot * stride + pos) * nbits;
+    return (slot * stride + planes_window_pos(a, p, 0)) * nbits;
+}
+DD_STAGE_FN uint32_t planes_lds_word(uint32_t first, uint32_t u, uint32_t nbits)
+{
+    return first + u * (DD_TDD_PLANES_T * nbits);
 }
 
 // Words a lane has for a window of P positions from sample a on.

@@ -28,7 +28,8 @@ static int window(uint32_t a, uint32_t P, uint32_t nbits, uint32_t slots, uint32
                 const uint32_t run = (a + pos) / T - 32 * (a / T / 32);  // from the start tile's first run on
                 if ((a + pos) % T != p || 32 * k + shift % 32 != run) bad |= 4;
                 if (k == 1 && shift % 32 && !third) bad |= 8;
-                const uint32_t word = planes_lds_word(slot, stride, pos, nbits);
+                const uint32_t word = planes_lds_word(planes_lds_first(slot, stride, a, p, nbits), u, nbits);
+                if (word != (slot * stride + pos) * nbits) bad |= 64;
                 if (word < slot * stride * nbits || word + nbits > (slot + 1) * stride * nbits) bad |= 16;
             });
         for (uint32_t i = 0; i < P; ++i) bad |= (seen[i] != 1) * 32;
