@@ -129,8 +129,9 @@ hipError_t dd_tdd_dedisperse_lds_batch(const dd_tdd_beam* beams, const uint32_t*
 #define DD_TDD_PLANES_SPL 64
 static inline int dd_tdd_tiling_is_planes(dd_tdd_tiling t) { return t.samples_per_lane == DD_TDD_PLANES_SPL; }
 // Whether the bit-plane kernel is expected to be the faster one for nout
-// outputs per DM (of all beams together) in ntiles tiles of 4096 (host only).
-int dd_tdd_planes_pay(unsigned nbits, size_t nchans, size_t ntiles, size_t nout, size_t ndm);
+// outputs per DM (of all beams together) in ntiles tiles of 4096, spread the
+// samples by which the delays of 16 DMs in a row differ at most (host only).
+int dd_tdd_planes_pay(unsigned nbits, size_t nchans, size_t ntiles, size_t nout, size_t ndm, size_t spread);
 unsigned dd_tdd_planes_chunk(unsigned nbits, size_t nact, unsigned dms_per_wave, unsigned waves);
 int dd_tdd_planes_tilings(unsigned nbits, dd_tdd_tiling* out, int max);
 hipError_t dd_tdd_transpose_planes(const uint8_t* in, size_t nsamps, size_t in_stride, unsigned nbits, size_t nchans,

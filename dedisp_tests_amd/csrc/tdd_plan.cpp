@@ -194,40 +194,68 @@ constexpr size_t kPlanesLds = 80 * 1024, kPlanesLdsOne = 158 * 1024;
 // 1- and 2-bit: from 96 of them on it is the faster one at any channel count
 // (96 to 560 workgroups, 16 to 256 ch: 1.2 to 3.3 times; 0.98 to 1.1 with two
 // tiles, the second half empty).
-// 4- and 8-bit gain less (1.7 and 1.4 times at most, 1024 ch) and lose it
-// where the channels are few or a last round of workgroups is nearly empty, so
-// both times are estimated: the planes' by rounds of 256 workgroups, two of
-// which share the CUs; the runs kernel's (4-bit) by its own rounds, three of
-// which do; the packed lanes' (8-bit) by the outputs. Fitted to 896 launches of
-// 16 to 1024 ch, 2 to 16 tiles and 96 to 2100 workgroups, within 6 % rms, and
-// taken with that to spare; below 48 ch the 4-bit estimates are too close to
-// each other to tell. Of those launches 4-bit takes 341 of 576, 8-bit 131 of
-// 320; a bound of 96 (8-bit: 448) workgroups took all of them and was slower by
-// more than 3 % on 122 and on 123, down to 0.67 (16 ch) and 0.71 (32 ch), where
-// these estimates are on 3 and on 3, down to 0.93 and 0.96. On 207 others drawn
-// at random the bound was slower on 35 of 143, the estimates on none of 79.
-extern "C" int dd_tdd_planes_pay(unsigned nbits, size_t nchans, size_t ntiles, size_t nout, size_t ndm)
+// 4- and 8-bit gain less and lose it where the channels are few or a last round
+// of workgroups is nearly empty, so both times are estimated (us), fitted to
+// launches of 16 to 1024 ch, 60 to 2500 workgroups and delays 0.2 to 330 samples
+// apart from DM to DM (2622 launches, within 9 % rms at the widest delays, 6 %
+// else): the planes' by rounds of 256 workgroups, two of which share the CUs
+// where two fit their LDS; the runs kernel's (4-bit) by its own rounds, three of
+// which do; the packed lanes' (8-bit) by the outputs. 4-bit planes take 2 DMs per
+// wave, 1 where the delays spread too far for that (twice the workgroups), and
+// then one workgroup per CU where they spread too far for two. Taken with a
+// margin for the estimates; below 48 ch the 4-bit ones are too close to tell.
+// 4-bit takes 1046 of 1759, 9 of them slower by more than 3 %, down to 0.93; a
+// bound of 96 workgroups was on 349, down to 0.67. 8-bit: 229 of 863 and 5, down
+// to 0.88; a bound of 448 on 211, down to 0.66.
+extern "C" int dd_tdd_planes_pay(unsigned nbits, size_t nchans, size_t ntiles, size_t nout, size_t ndm, size_t spread)
 {
     const dd_tdd_tiling t = default_tiling(nbits);
     if (!dd_tdd_tiling_is_planes(t)) return 0;
-    const size_t dpb = (size_t)t.dms_per_wave * t.waves;
-    const size_t wgs = ntiles * div_up(ndm, dpb), rounds = div_up(wgs, size_t(256));
-    if (nbits <= 2) return wgs >= 96;
     const double n = (double)nchans, out = (double)nout * (double)ndm * 1e-6;
-    if (nbits == 4) {  // us
-        const size_t runs = div_up(div_up(nout, size_t(7 * 256)) * div_up(ndm, size_t(16)), size_t(256));
-        const double part[3] = {0.0, 9.3 + 0.211 * n, 10.1 + 0.286 * n};
-        const double planes = 29.8 + 0.067 * n + 0.152 * out + (12.9 + 0.342 * n) * (double)(rounds / 2) +
-                              (7.7 + 0.215 * n) * (double)(rounds % 2);
-        const double other = 21.2 + 0.083 * n + 0.046 * out + (11.9 + 0.381 * n) * (double)(runs / 3) + part[runs % 3];
-        return nchans >= 48 && 1.04 * planes < other;
+    if (nbits <= 2) return ntiles * div_up(ndm, size_t(16)) >= 96;
+    if (nbits == 8) {
+        const size_t rounds = div_up(ntiles * div_up(ndm, size_t(8)), size_t(256));
+        const double planes = 30.4 + (3.8 + 0.24 * n) * std::max((double)rounds, 1.4);
+        const double other = 21.4 + 0.147 * n + (0.459 + 0.0339 * n) * out;
+        return 1.06 * planes < other;
     }
-    const double planes = 30.4 + (3.8 + 0.24 * n) * std::max((double)rounds, 1.4);
-    const double other = 21.4 + 0.147 * n + (0.459 + 0.0339 * n) * out;
-    return 1.06 * planes < other;
+    const auto lds = [](size_t samples) {
+        return (4 * round_up(DD_TDD_PLANES_T + samples, 64) + DD_TDD_PLANES_T) * 4 * 4;
+    };
+    const size_t half = spread * 7 / 15;  // of 8 DMs
+    const bool two_dms = lds(spread) <= kPlanesLds, shared = two_dms || lds(half) <= kPlanesLds;
+    if (nchans < 48 || lds(half) > kPlanesLdsOne) return 0;
+    const size_t r = div_up(ntiles * div_up(ndm, size_t(two_dms ? 16 : 8)), size_t(256));
+    const size_t runs = div_up(div_up(nout, size_t(7 * 256)) * div_up(ndm, size_t(16)), size_t(256));
+    const double pairs = (double)(r / 2), odd = (double)(r % 2), wide = n * (double)spread * 1e-3;
+    double planes;
+    if (two_dms)
+        planes = 26.6 + 0.048 * n + 0.282 * out + (15.2 + 0.347 * n) * pairs + (10.6 + 0.227 * n) * odd +
+                 0.0662 * wide * (double)r;
+    else if (shared)
+        planes = 27.0 + 0.057 * n + 0.195 * out + (10.1 + 0.172 * n) * pairs + (6.3 + 0.138 * n) * odd +
+                 0.04 * wide * (double)r;
+    else
+        planes = 26.5 + 0.028 * n + 0.1 * out + (8.0 + 0.21 * n) * (double)r + 0.0225 * wide * (double)r;
+    const double part[3] = {0.0, 10.3 + 0.224 * n, 10.6 + 0.29 * n};
+    const double other = 21.0 + 0.059 * n + 0.188 * out + (12.0 + 0.377 * n) * (double)(runs / 3) + part[runs % 3] +
+                         (0.0645 + 0.0325 * (double)runs) * wide;
+    return 1.03 * planes < other;
 }
 
 namespace {
+
+// Samples by which the delays of 16 DMs in a row differ at most, delay the
+// largest of the delay table (samples per unit DM).
+size_t dm_spread(const float* dms, size_t count, float delay)
+{
+    float widest = 0.f;
+    for (size_t i = 0; i < count; i += 16) {
+        const auto ends = std::minmax_element(dms + i, dms + std::min(count, i + 16));
+        widest = std::max(widest, *ends.second - *ends.first);
+    }
+    return (size_t)std::min(std::max((double)widest * delay, 0.0), 1e9);
+}
 
 // Output samples per time tile of the channel-sum kernel: 7 runs of 256 for
 // the runs-layout kernel, 32 for the bit-plane kernel, 64 lanes x
@@ -729,7 +757,8 @@ void TDDPlan::execute_span(size_type nsamps, const byte_type* in, size_type in_n
     const unsigned nbits = (unsigned)in_nbits;
     prepare_tables(nbits, first_dm_idx, dm_count, true,
                    !m_state->tuned[nbits].waves &&
-                       !dd_tdd_planes_pay(nbits, m_nchans, planes_tiles(nsc), nsc, dm_count));
+                       !dd_tdd_planes_pay(nbits, m_nchans, planes_tiles(nsc), nsc, dm_count,
+                                          dm_spread(h_dm_list.data() + first_dm_idx, dm_count, h_delay_table.back())));
     st.row_words = row_words_for(nbits, nsamps, nsc);
 
     // ---- input ----
@@ -901,7 +930,8 @@ void TDDPlan::execute_noalloc(size_type nsamps, const byte_type* in, size_type i
     // layout (and its tables) may, and is kept for the series length
     const std::array<uint64_t, 3> packed_key = {m_tables_version, nbits, nsamps};
     const bool few = !st.tuned[nbits].waves &&
-                     !dd_tdd_planes_pay(nbits, m_nchans, planes_tiles(nsc), nsc, m_dm_count);
+                     !dd_tdd_planes_pay(nbits, m_nchans, planes_tiles(nsc), nsc, m_dm_count,
+                                        dm_spread(h_dm_list.data(), m_dm_count, h_delay_table.back()));
     if (few || st.noalloc_packed == packed_key) {
         if (!lay_out(true)) DD_THROW(DEDISP_MEM_ALLOC_FAILED);
     } else if (!lay_out(false)) {
@@ -984,7 +1014,9 @@ void TDDPlan::execute_batch(size_type nbeams, const size_type* nsamps, const byt
         outputs += nsamps[b] - m_max_delay;
     }
     prepare_tables(nbits, 0, m_dm_count, true,
-                   !st.tuned[nbits].waves && !dd_tdd_planes_pay(nbits, m_nchans, tiles, outputs, m_dm_count));
+                   !st.tuned[nbits].waves &&
+                       !dd_tdd_planes_pay(nbits, m_nchans, tiles, outputs, m_dm_count,
+                                          dm_spread(h_dm_list.data(), m_dm_count, h_delay_table.back())));
     if (!st.fast || st.nact == 0) {
         // weighted killmask or 16/32-bit samples: one beam after another
         for (size_t b = 0; b < nbeams; ++b)

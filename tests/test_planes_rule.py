@@ -8,8 +8,8 @@ import pytest
 def pays(dd):
     fn = dd.lib().dd_tdd_planes_pay
     fn.restype = C.c_int
-    fn.argtypes = [C.c_uint] + [C.c_size_t] * 4
-    return lambda nbits, nch, nout, ndm: bool(fn(nbits, nch, -(-nout // 4096), nout, ndm))
+    fn.argtypes = [C.c_uint] + [C.c_size_t] * 5
+    return lambda nbits, nch, nout, ndm, step=2: bool(fn(nbits, nch, -(-nout // 4096), nout, ndm, int(15 * step)))
 
 
 # times on the other kernels and on bit planes (us)
@@ -33,6 +33,18 @@ def test_launches_that_bit_planes_slow_down_stay_off_them(pays, nbits, nch, nout
 ])
 def test_launches_that_bit_planes_speed_up_take_them(pays, nbits, nch, nout, ndm, other, planes):
     assert planes < other and pays(nbits, nch, nout, ndm)
+
+
+# delays step samples apart from DM to DM
+@pytest.mark.parametrize("nch,nout,ndm,step,other,planes", [
+    (512, 109686, 58, 255.6, 401, 201), (512, 4460, 939, 323.0, 511, 230), (1000, 89900, 81, 163.6, 644, 330),
+    (328, 99619, 184, 88.3, 252, 194), (200, 65470, 91, 75.5, 110, 87), (512, 11420, 491, 124.2, 266, 173),
+    (200, 8237, 2422, 165.1, 195, 292), (200, 12397, 2361, 169.4, 302, 352), (96, 83165, 1190, 256.5, 495, 527),
+    (200, 47188, 2296, 157.4, 808, 877),
+])
+def test_wide_windows(pays, nch, nout, ndm, step, other, planes):
+    """1 DM per wave, and one workgroup per CU, where the windows need it."""
+    assert pays(4, nch, nout, ndm, step) == (planes < other)
 
 
 @pytest.mark.parametrize("nbits", [1, 2, 4, 8, 16, 32])
