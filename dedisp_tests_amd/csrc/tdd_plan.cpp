@@ -192,8 +192,8 @@ constexpr size_t kPlanesLds = 80 * 1024, kPlanesLdsOne = 158 * 1024;
 // The bit-plane kernel's workgroups are larger (4096 outputs) and fewer than
 // the other kernels', so they leave more of the chip idle where there are few.
 // 1- and 2-bit: from 96 of them on it is the faster one at any channel count
-// (96 to 560 workgroups, 16 to 256 ch: 1.2 to 3.3 times; 0.98 to 1.1 with two
-// tiles, the second half empty).
+// (16 to 1024 ch: 1.3 to 3.5 times and 1.0 to 3.1; of 447 2-bit launches 7 were
+// slower, with the second of two tiles nearly empty, down to 0.76).
 // 4- and 8-bit gain less and lose it where the channels are few or a last round
 // of workgroups is nearly empty, so both times are estimated (us), fitted to
 // launches of 16 to 1024 ch, 60 to 2500 workgroups and delays 0.2 to 330 samples
@@ -206,7 +206,8 @@ constexpr size_t kPlanesLds = 80 * 1024, kPlanesLdsOne = 158 * 1024;
 // margin for the estimates; below 48 ch the 4-bit ones are too close to tell.
 // 4-bit takes 1046 of 1759, 9 of them slower by more than 3 %, down to 0.93; a
 // bound of 96 workgroups was on 349, down to 0.67. 8-bit: 229 of 863 and 5, down
-// to 0.88; a bound of 448 on 211, down to 0.66.
+// to 0.88; a bound of 448 on 211, down to 0.66. (On 530 more, not fitted to:
+// 4-bit 2 of 194, 8-bit none of 33; the bounds 76 and 29.)
 extern "C" int dd_tdd_planes_pay(unsigned nbits, size_t nchans, size_t ntiles, size_t nout, size_t ndm, size_t spread)
 {
     const dd_tdd_tiling t = default_tiling(nbits);
