@@ -175,8 +175,7 @@ struct Geo {
 // WAVES waves per workgroup, each MT 16-row DM tiles (sharing every B read);
 // NS bin slots (with MIRROR NS/2 direct bins and their mirrors).
 //
-// PIPE (bfloat16 and float16 with the delays computed in the kernel, 8 waves
-// of 2 DM tiles): software pipelined. A K-step is NDIR units, one computed bin
+// PIPE (the delays computed in the kernel, 8 waves of 2 DM tiles): software pipelined. A K-step is NDIR units, one computed bin
 // each (its direct slot and, with MIRROR, its mirror slot); between the
 // product groups of a unit the wave generates pieces of the next unit's
 // phasors (the next K-step's first bin in the last unit) and stages half of

@@ -551,8 +551,8 @@ bool contraction_packs(const FDDState& st)
 }
 
 // Whether the spectra and the packed output use the bin-block layout (the
-// pipelined float16 / bfloat16 contraction with mirror bins and the packed
-// output, nfft <= 65536): a workgroup of the contraction then reads and
+// pipelined contraction with mirror bins and the packed output, nfft <=
+// 65536): a workgroup of the contraction then reads and
 // writes whole cache lines (DEDISP_FDD_BLOCKED=0 keeps rows of Xp / Yp).
 bool blocked_layout(const FDDState& st, size_t nfft, size_t nchunk, size_t Xp)
 {
@@ -751,7 +751,7 @@ void FDDGPUPlan::execute_fdd(size_type nsamps, const byte_type* in, size_type in
         d_out = st.d_out.as<float>();
     }
     // DEDISP_FDD_VALU=1 selects the float32 vector-ALU contraction instead of
-    // the matrix cores (same arithmetic as the float32 MFMA form)
+    // the matrix cores
     for (size_t b0 = 0; b0 < ndm; b0 += dm_batch) {
         const size_t nb = std::min(dm_batch, ndm - b0);
         ctx.timer.begin(StageTimer::DEDISPERSE, stream);

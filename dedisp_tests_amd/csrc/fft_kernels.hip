@@ -88,7 +88,7 @@ struct FftShape {
     static constexpr int LDS_FLOATS = X1 > X2 ? X1 : X2;
 };
 
-// Bin-block layout of the real spectra (the float16 / bfloat16 matrix-core
+// Bin-block layout of the real spectra (the matrix-core
 // contraction with mirror bins reads and writes it): bins k and k+1 (k even,
 // k <= M/2) and their mirrors M-k, M-k-1 form block k/2, the four values of a
 // block for every chunk contiguous, so a workgroup of the contraction reads

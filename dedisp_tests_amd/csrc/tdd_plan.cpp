@@ -166,7 +166,7 @@ dd_tdd_tiling packed_tiling(unsigned nbits)
 
 // Bit planes (tdd_planes.hip) for every sub-byte width and, 1 DM per wave for
 // its 18 counter planes, 8-bit: 1-bit, 512 ch x 200003 x 501 DMs 1.07 -> 0.38
-// ms per execute; 2-bit, 512 ch x 4 beams x 1024 DMs 21.8 -> 8.3 ms; 4-bit,
+// ms per execute; 2-bit, 512 ch x 4 beams x 1024 DMs 21.8 -> 8.4 ms; 4-bit,
 // 1024 ch x 2^20 x 1167 DMs 22.8 -> 14.6 ms (runs layout before); 8-bit, 1024
 // ch x 15625 x 3000 DMs 1.92 -> 1.43 ms.
 dd_tdd_tiling default_tiling(unsigned nbits)
