@@ -609,12 +609,14 @@ extern "C" hipError_t dd_tdd_dedisperse_planes(const uint32_t* rows, size_t row_
 extern "C" int dd_tdd_planes_tilings(unsigned nbits, dd_tdd_tiling* out, int max)
 {
     int n = 0;
+    dd_tdd_tiling shapes[8];  // (fewer per width)
 #define DD_LIST(NB, CC, PL, DPW, W)                                                                     \
     if (nbits == NB) {                                                                                  \
         bool seen = false;                                                                              \
-        for (int k = 0; k < n && k < max && out; ++k) seen |= out[k].dms_per_wave == DPW && out[k].waves == W; \
+        for (int k = 0; k < n; ++k) seen |= shapes[k].dms_per_wave == DPW && shapes[k].waves == W;      \
         if (!seen) {                                                                                    \
-            if (n < max && out) out[n] = dd_tdd_tiling{DD_TDD_PLANES_SPL, DPW, W, 16, 0};               \
+            shapes[n] = dd_tdd_tiling{DD_TDD_PLANES_SPL, DPW, W, 16, 0};                                \
+            if (n < max && out) out[n] = shapes[n];                                                     \
             ++n;                                                                                        \
         }                                                                                               \
     }

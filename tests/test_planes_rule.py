@@ -52,3 +52,18 @@ def test_smallest_launches_and_wide_samples(pays, nbits):
     assert not pays(nbits, 64, 1, 1) and not pays(nbits, 1024, 4096, 16)
     if nbits > 8:
         assert not pays(nbits, 1024, 1 << 20, 2048)
+
+
+@pytest.mark.parametrize("nbits,planes", [(1, 2), (2, 2), (4, 2), (8, 1)])
+def test_tilings_are_counted_as_they_are_listed(dd, nbits, planes):
+    """Without a buffer, with one too short and with one that holds them all."""
+    for name in ("dd_tdd_planes_tilings", "dd_tdd_lds_tilings"):
+        fn = getattr(dd.lib(), name)
+        fn.restype, fn.argtypes = C.c_int, [C.c_uint, C.c_void_p, C.c_int]
+        buf = (C.c_uint * (5 * 64))()
+        n = fn(nbits, buf, 64)
+        assert fn(nbits, None, 0) == n and fn(nbits, (C.c_uint * 5)(), 1) == n
+        shapes = [tuple(buf[5 * i : 5 * i + 4]) for i in range(n)]
+        assert len(set(shapes)) == n and sum(s[0] == 64 and s[2] == 8 for s in shapes) >= planes
+        if name == "dd_tdd_planes_tilings":
+            assert n == planes
