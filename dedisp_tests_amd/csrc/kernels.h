@@ -127,6 +127,7 @@ hipError_t dd_tdd_dedisperse_lds_batch(const dd_tdd_beam* beams, const uint32_t*
 // wstart)/32T + 2 tiles.
 #define DD_TDD_PLANES_T 128
 #define DD_TDD_PLANES_SPL 64
+#define DD_TDD_PLANES_LDS_MAX (158 * 1024)  // bytes of LDS a workgroup takes at most
 static inline int dd_tdd_tiling_is_planes(dd_tdd_tiling t) { return t.samples_per_lane == DD_TDD_PLANES_SPL; }
 // Whether the bit-plane kernel is expected to be the faster one for nout
 // outputs per DM (of all beams together) in ntiles tiles of 4096, spread the

@@ -185,7 +185,7 @@ constexpr size_t kLdsBudget = 64 * 1024;  // bytes of LDS per workgroup
 // 0.55 ms with 1 DM per wave, 0.69 with 2 in one workgroup per CU, 1.35 on
 // packed lanes; 4-bit 1.07, 1.31, 1.31. 8-bit with one workgroup per CU lost to
 // the packed lanes, 2.60 against 2.16 ms.
-constexpr size_t kPlanesLds = 80 * 1024, kPlanesLdsOne = 158 * 1024;
+constexpr size_t kPlanesLds = 80 * 1024, kPlanesLdsOne = DD_TDD_PLANES_LDS_MAX;
 
 }  // namespace
 

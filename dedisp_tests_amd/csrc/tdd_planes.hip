@@ -590,9 +590,11 @@ extern "C" hipError_t dd_tdd_dedisperse_planes(const uint32_t* rows, size_t row_
         if ((nact + 2 * CC - 1) / (2 * CC) * 2 != nchunk) return hipErrorInvalidValue;                          \
         const size_t bytes = ((size_t)CC * tl.window_words + T) * NB * 4;                                             \
         auto kern = tdd_planes_k<NB, CC, PL, DPW, W>;                                                           \
+        if (bytes > DD_TDD_PLANES_LDS_MAX) return hipErrorInvalidValue;                                         \
         if (bytes > 64 * 1024) {                                                                                \
+            /* the same limit from every thread: one plan's must not end below what another's is launched with */ \
             hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,   \
-                                               (int)bytes);                                                     \
+                                               DD_TDD_PLANES_LDS_MAX);                                          \
             if (e != hipSuccess) return e;                                                                      \
         }                                                                                                       \
         hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(W * 64), bytes, stream, rows, row_words, code,   \

@@ -707,3 +707,41 @@ def test_tdd_rows_of_odd_bytes_in_a_padded_stride(dd, orc, monkeypatch, nbits, n
     delays = orc.delay_table(nch, *[f32(g) for g in geom])
     assert np.array_equal(out.cpu().numpy(), orc.tdd(nch, delays, None, dms, n, md, data, nbits, 32))
     plan.close()
+
+
+def test_tdd_planes_windows_of_different_plans_in_threads(dd, orc, monkeypatch):
+    """Plans whose windows take 80 to 158 KB of LDS of the same kernel, executed
+    from a thread each at the same time."""
+    import threading
+    import torch
+    monkeypatch.setenv("DEDISP_TDD_TILING", "64,2,8,16")
+    nch, nbits, geom = 40, 4, (64e-6, 1500.0, -10.0)
+    delays = orc.delay_table(nch, *[f32(g) for g in geom])
+    jobs = []
+    for step in (160, 250, 330):
+        plan = dd.Plan(nch, *geom, impl=dd.TDD)
+        dms = (np.arange(24) * (step / float(delays[-1]))).astype(f32)
+        plan.set_dm_list(dms)
+        n = 4200 + plan.max_delay
+        s = np.random.default_rng(step).integers(0, 1 << nbits, size=(n, nch)).astype(np.uint8)
+        data = dd.pack_samples(s, nbits)
+        out = torch.empty((24, 4200), dtype=torch.float32, device="cuda")
+        jobs.append((plan, n, torch.from_numpy(data).cuda(), out, orc.tdd(nch, delays, None, dms, n, plan.max_delay, data, nbits, 32)))
+    torch.cuda.synchronize()
+    errors = []
+
+    def work(plan, n, d_in, out, ref):
+        for _ in range(50):
+            errors.append(plan.execute_raw(n, d_in, nbits, out, 32, dd.DEVICE_POINTERS))
+
+    threads = [threading.Thread(target=work, args=j) for j in jobs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert errors == [0] * 150
+    for plan, n, d_in, out, ref in jobs:
+        assert _shape(plan) == (64, 1, 8)
+        assert np.array_equal(out.cpu().numpy(), ref)
+        plan.close()
